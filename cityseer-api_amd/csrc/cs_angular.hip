@@ -1,4 +1,7 @@
-// cs_angular.hip -- simplest-path (angular) centrality on the dual graph.
+// cs_angular.hip -- simplest-path (angular) centrality on the dual graph, one
+// lane per source: what the LDS search (cs_angwave.hip) does not take or has no
+// room for (tolerances above the tie band, searches of thousands of nodes,
+// negative increments), the single-source tree and the reach lists.
 //
 // Angular route increments are turn angles plus 1e-6 x length
 // (centrality.rs:665-667): straight continuations cost almost nothing, so no
@@ -1275,8 +1278,18 @@ void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<u
   const int dev0 = specs[0].dg->device;
   int n_cu = 0;
   hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev0), "attribute");
+  if ((explicit_items ? explicit_items->size() : n_implicit) == 0) return;
+  // one wave per source with its search in LDS; what does not fit there (or a
+  // launch it does not take) searches with one lane per source below
+  bool done = false;
+  std::vector<uint2> rest;
+  if (!default_tuning().ang_lanes) rest = launch_simplest_wave(specs, explicit_items, n_implicit, stream, st, progress, &done);
+  if (done) {
+    if (rest.empty()) return;
+    st.retries += (uint32_t)rest.size();
+    explicit_items = &rest;
+  }
   const uint32_t n_real = explicit_items ? (uint32_t)explicit_items->size() : n_implicit;
-  if (n_real == 0) return;
   const uint32_t per_wave = sources_per_wave(n_real, 4u * (uint32_t)n_cu);
   std::vector<uint2> items;
   if (explicit_items) {
@@ -1654,6 +1667,7 @@ std::vector<uint32_t> launch_reach_simplest(Graph &g, DevGraph &dg, DevEdges &de
 }
 
 void release_angular_workspaces() {
+  release_angular_wave_workspaces();
   std::lock_guard<std::mutex> lk(g_ang_mu);
   for (auto &dv : g_ang) {
     AngWorkspace &w = *dv.second;

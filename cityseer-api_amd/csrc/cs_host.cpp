@@ -170,6 +170,7 @@ void free_edges(DevEdges &d) {
   (void)hipFree(d.fwd_eid);
   (void)hipFree(d.ang_adj);
   (void)hipFree(d.ang_srow);
+  if (d.ang_wave) free_angular_wave(*d.ang_wave);
 }
 
 }  // namespace
@@ -197,7 +198,7 @@ void set_node_order_from_xy(Graph &g, const double *x, const double *y) {
   if (!g.dev.empty() || g.order_frozen)
     fail(CS_EINVAL, "node coordinates must be set before the graph's first computation");
   const uint32_t n = g.n;
-  if (g.is_dual || n < 2) return;  // dual graphs keep their order (angular search)
+  if (n < 2) return;
   double x0 = INFINITY, x1 = -INFINITY, y0 = INFINITY, y1 = -INFINITY;
   for (uint32_t i = 0; i < n; ++i) {
     if (!std::isfinite(x[i]) || !std::isfinite(y[i])) return;  // no usable layout: keep the given order
@@ -214,6 +215,16 @@ void set_node_order_from_xy(Graph &g, const double *x, const double *y) {
     key[i] = {hilbert_index(qx, qy), i};
   }
   std::sort(key.begin(), key.end());
+  if (g.is_dual) {
+    // dual graphs keep their order, but for the LDS angular search
+    g.ang_iperm.resize(n);
+    g.ang_perm.resize(n);
+    for (uint32_t d = 0; d < n; ++d) {
+      g.ang_iperm[d] = key[d].second;
+      g.ang_perm[key[d].second] = d;
+    }
+    return;
+  }
   g.identity_order = true;
   for (uint32_t d = 0; d < n; ++d) {
     g.iperm[d] = key[d].second;

@@ -44,6 +44,52 @@ struct DevMem {
   DevMem &operator=(const DevMem &) = delete;
 };
 
+// Grow-only device buffer.
+struct DevVec {
+  void *p = nullptr;
+  size_t bytes = 0;
+  void *get(size_t need, const char *what) {
+    if (need > bytes) {
+      if (p) hip_check(hipFree(p), "hipFree");
+      p = nullptr;
+      bytes = 0;
+      if (hipMalloc(&p, need) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        fail(CS_ENOMEM, std::string("could not allocate ") + std::to_string(need >> 20) + " MiB of " + what);
+      }
+      bytes = need;
+    }
+    return p;
+  }
+  void release() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+  }
+};
+
+// What the LDS angular search (cs_angwave.hip) reads of a dual graph, nodes in
+// an order of its own (along a Hilbert curve of their coordinates).
+struct AngWaveGraph {
+  bool usable = false;  // increments and seconds finite and non-negative, rows and page tables within its limits
+  uint4 *row = nullptr;
+  float *row_wm = nullptr;
+  uint4 *spill = nullptr;
+  float *spill_wm = nullptr;
+  float *wm = nullptr;
+  uint32_t *perm = nullptr, *orig = nullptr;
+  float max_w = 0.0f;
+  // nodes and runs of 2^k nodes (k < 10) that searches up to a time limit reach:
+  // the most over a few probed sources, per limit asked for so far
+  struct Reach {
+    uint32_t nodes = 0;
+    uint32_t pages[10] = {0};
+    bool chains = false;  // most nodes lead on to others (streets cut into short pieces)
+  };
+  std::map<float, Reach> reach;
+};
+
 // Speed-dependent device edge arrays for one (device, speed).
 struct DevEdges {
   float speed = 0.0f;
@@ -65,6 +111,7 @@ struct DevEdges {
   uint4 *ang_srow = nullptr;  // [2N][4] usable out-edges of each dual state (cs_angular.hip)
   float min_es_ang = 0.0f;
   float max_w_ang = 0.0f;  // largest route increment (angle + 1e-6 length) of the dual's edges
+  std::unique_ptr<AngWaveGraph> ang_wave;
 };
 
 struct DevGraph {
@@ -106,6 +153,8 @@ struct Graph {
   // its inverse; both identity otherwise. Every entry point translates.
   std::vector<uint32_t> perm, iperm;
   bool identity_order = true;
+  // The LDS angular search's own order of a dual's nodes (empty: as given).
+  std::vector<uint32_t> ang_perm, ang_iperm;
   mutable std::atomic<bool> order_frozen{false};  // set once an entry point has translated ids
 
   std::mutex mu;
@@ -340,6 +389,15 @@ struct AngSpec {
 // {job, source position} (or, without a list, sources 0..n_implicit-1 of job 0).
 void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items,
                           uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress = nullptr);
+
+// The same with each source's whole search in the LDS of one wave
+// (cs_angwave.hip), where every request allows it (`done` false: none ran).
+// Returns the items whose search did not fit, which have added nothing.
+std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items,
+                                        uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress,
+                                        bool *done);
+void free_angular_wave(AngWaveGraph &w);
+void release_angular_wave_workspaces();
 
 void launch_simplest(Graph &g, DevGraph &dg, DevEdges &de, const CallSpec &cs,
                      const uint32_t *d_sources, const float *d_wt, uint32_t n_sources,

@@ -30,14 +30,10 @@
 //    in reverse (centrality.rs:823-873), reading the predecessor's slot that
 //    the forward fold stored.
 #include "cs_internal.hpp"
+#include "cs_wave.hpp"
 
 #include <algorithm>
 
-// 64-bit wave reductions of the device library (declared by HIP only under an
-// opt-in macro).
-extern "C" __device__ uint32_t __ockl_wfscan_add_u32(uint32_t, bool);
-extern "C" __device__ __attribute__((const)) unsigned long long __ockl_wfred_add_u64(unsigned long long);
-extern "C" __device__ __attribute__((const)) double __ockl_wfred_add_f64(double);
 #include <cmath>
 #include <cstring>
 
@@ -47,7 +43,6 @@ namespace {
 
 constexpr uint32_t kFailCap = 1u, kFailBucket = 2u, kFailRing = 4u, kFailInternal = 8u, kFailWide = 16u;
 constexpr int kChunk = 1;           // in-edges per lane per step of the segment closeness walk
-constexpr uint32_t kXcd = 8;   // XCDs; workgroups are dealt to them round-robin
 constexpr uint32_t kScanQ = 4;     // key words per lane per step of the node-ordered result flush
 constexpr uint32_t kFlushList = kScanQ * 64;  // LDS list of one flush step (reached nodes, index order)
 constexpr uint32_t kFlushWords = 3 * kFlushList;  // {node, seconds bits, slot} per list entry
@@ -136,62 +131,6 @@ struct SearchArgs {
 // magnify; the f64 exponential rounded to f32 agrees with the correctly
 // rounded value except when it lands within 2^-29 of a rounding boundary.
 __device__ __forceinline__ float exp_f32(float x) { return (float)exp((double)x); }
-
-// Wave-private workspace: only the owning wave reads or writes it, so
-// workgroup scope (coherent in the CU's L1 and the XCD's L2) is sufficient.
-__device__ __forceinline__ uint64_t ld64(const uint64_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ uint32_t ld32(const uint32_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ double ldd(const double *p) {
-  return __longlong_as_double((long long)ld64(reinterpret_cast<const uint64_t *>(p)));
-}
-__device__ __forceinline__ void st32(uint32_t *p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void st64(uint64_t *p, uint64_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void std_(double *p, double v) {
-  st64(reinterpret_cast<uint64_t *>(p), (uint64_t)__double_as_longlong(v));
-}
-__device__ __forceinline__ uint64_t wmax64(uint64_t *p, uint64_t v) {
-  return __hip_atomic_fetch_max(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void wadd_f64(double *p, double v) {
-  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-// LDS ring counters (one wave's private row).
-__device__ __forceinline__ uint32_t lds_ld(const uint32_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void lds_st(uint32_t *p, uint32_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ uint32_t lds_add(uint32_t *p, uint32_t v) {
-  return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-// Results shared by all waves (accumulators): device scope.
-__device__ __forceinline__ void gadd_f64(double *p, double v) { unsafeAtomicAdd(p, v); }
-// Orders this wave's earlier memory operations before its later ones (all lanes).
-__device__ __forceinline__ void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-__device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
-__device__ __forceinline__ uint32_t rank_below(uint64_t m) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-// Wave-wide reductions over the active lanes (the device library's DPP
-// sequences: no LDS round trips), result in every lane.
-__device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return __ockl_wfred_add_u32(v); }
-__device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) { return __ockl_wfred_add_u64(v); }
-__device__ __forceinline__ double wave_sum(double v) { return __ockl_wfred_add_f64(v); }
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ uint32_t wave_or(uint32_t v) { return __ockl_wfred_or_u32(v); }
 
 // Node key, one 64-bit word: epoch (9 bits) | settled (1) | low 31 bits of the
 // complemented f32 seconds (31; seconds are never negative, so the dropped top
@@ -1939,31 +1878,6 @@ float choose_delta(const Graph &g, const DevEdges &de, float maxsec, bool &exact
   }
   return (float)delta;
 }
-
-// Grow-only device buffer.
-struct DevVec {
-  void *p = nullptr;
-  size_t bytes = 0;
-  void *get(size_t need, const char *what) {
-    if (need > bytes) {
-      if (p) hip_check(hipFree(p), "hipFree");
-      p = nullptr;
-      bytes = 0;
-      if (hipMalloc(&p, need) != hipSuccess) {
-        (void)hipGetLastError();
-        p = nullptr;
-        fail(CS_ENOMEM, std::string("could not allocate ") + std::to_string(need >> 20) + " MiB of " + what);
-      }
-      bytes = need;
-    }
-    return p;
-  }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    bytes = 0;
-  }
-};
 
 struct Workspace {
   int device = -1;

@@ -1,0 +1,71 @@
+"""GPU: the LDS angular search where it could go wrong, against the oracle: exactly equal routes
+everywhere (one at a time, and many at one route), streets cut into short straight pieces (no two
+states safe together), crossings of more than four streets (longer rows than one state's lanes),
+more thresholds than one back-propagation pass holds, and searches that outgrow the room the
+probed sources asked for (a dense knot in a sparse network)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cityseer import _native
+from cityseer.tools import mock
+import oracle.oracle as O
+from oracle.oracle import OracleGraph
+from test_gpu_shortest import assert_close, say, stack
+
+pytestmark = pytest.mark.gpu
+
+SIMPLEST = ("node_density", "node_farness", "node_harmonic", "node_betweenness")
+
+
+def _grid(side):
+    """Unjittered square grid: every turn 0 or 90 degrees, every length 100."""
+    return mock.perturbed_lattice(side, jitter=0.0, drop_frac=0.0, len_range=(1.0, 1.0), seed=0)
+
+
+def _star(arms, rings, jitter):
+    """`arms` radial streets through one crossing, joined by rings: a crossing of `arms` streets."""
+    rng = np.random.default_rng(arms)
+    ang = 2 * np.pi * (np.arange(arms) + jitter * rng.uniform(-0.3, 0.3, arms)) / arms
+    x, y, edges = [0.0], [0.0], []
+    for r in range(1, rings + 1):
+        for a in range(arms):
+            x.append(100.0 * r * np.cos(ang[a]))
+            y.append(100.0 * r * np.sin(ang[a]))
+            me = 1 + (r - 1) * arms + a
+            edges.append((0 if r == 1 else me - arms, me))
+            edges.append((me, 1 + (r - 1) * arms + (a + 1) % arms))
+    x, y, edges = np.array(x), np.array(y), np.array(edges)
+    length = np.hypot(x[edges[:, 1]] - x[edges[:, 0]], y[edges[:, 1]] - y[edges[:, 0]]).astype(np.float32)
+    return mock.Lattice(x=x, y=y, edges=edges, length=length)
+
+
+def _knot():
+    """A lattice at 100 m with one 9 x 9 lattice at 4 m hung on its corner: the searches there reach
+    several times as many nodes as the rest."""
+    a, b = mock.perturbed_lattice(40, seed=5), mock.perturbed_lattice(9, spacing=4.0, jitter=1.0, seed=6)
+    k = len(a.x)
+    return mock.Lattice(x=np.concatenate([a.x, b.x + a.x[0] - 100.0]), y=np.concatenate([a.y, b.y + a.y[0] - 100.0]),
+                        edges=np.concatenate([a.edges, b.edges + k, [[0, k]]]),
+                        length=np.concatenate([a.length, b.length, [np.float32(60.0)]]).astype(np.float32))
+
+
+@pytest.mark.parametrize("name,distances", [
+    ("grid", [400, 900]), ("star8", [300, 700]), ("star9 even", [250, 600]), ("pieces", [150, 400, 700]),
+    ("five", [200, 300, 400, 500, 600]), ("one", [350]), ("knot", [150, 300])])
+def test_matches_oracle(name, distances):
+    O.set_heap_mode(False)
+    primal = {"grid": lambda: _grid(9), "star8": lambda: _star(8, 4, 1.0), "star9 even": lambda: _star(9, 3, 0.0),
+              "pieces": lambda: mock.decompose_lattice(mock.perturbed_lattice(8, seed=71), 15.0),
+              "five": lambda: mock.perturbed_lattice(12, seed=72, diag_frac=0.2),
+              "one": lambda: mock.perturbed_lattice(5, seed=73), "knot": _knot}[name]()
+    ns = mock.network_structure_from_lattice(mock.lattice_dual(primal))
+    say(f"angular search, {name}: {ns.node_count()} dual nodes, {distances} m")
+    got = stack(ns.centrality_simplest(distances=distances), SIMPLEST, distances)
+    ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest(distances)
+    assert np.array_equal(got[0], ref[0])
+    assert_close(got, ref, name)
+    if name == "knot":
+        assert _native.last_stats()["retries"] > 0
