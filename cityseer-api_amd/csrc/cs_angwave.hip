@@ -1200,6 +1200,10 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
                                         bool *done) {
   *done = false;
   const int dev = specs[0].dg->device;
+  // (also guards what the device's graphs keep for this search: a served slice
+  // comes without the graph's own lock)
+  WaveWorkspace &ws = wave_ws(dev);
+  std::lock_guard<std::mutex> lk(ws.mu);
   const uint32_t cap = default_tuning().cap;
   uint32_t N = 1, T = 1, maxp = 1, nodes = 0;
   uint32_t pages[10] = {0};
@@ -1242,8 +1246,6 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
   std::vector<uint2> items;
   if (explicit_items) items = *explicit_items;
   uint32_t n_list = explicit_items ? (uint32_t)items.size() : n_implicit;
-  WaveWorkspace &ws = wave_ws(dev);
-  std::lock_guard<std::mutex> lk(ws.mu);
   if (!ws.e0) {
     hip_check(hipEventCreate(&ws.e0), "event");
     hip_check(hipEventCreate(&ws.e1), "event");
