@@ -90,6 +90,22 @@ struct AngWaveGraph {
   std::map<float, Reach> reach;
 };
 
+// What the LDS shortest search (cs_disc.hip) reads of a graph.
+struct DiscGraph {
+  bool usable = false;
+  uint4 *row = nullptr;  // [N][blocks][4] in- and out-edge of each neighbour, device node order
+  uint32_t blocks = 1, maxp = 1;
+  std::vector<uint64_t> spans;  // nodes by their shortest in-edge (powers of two of a millisecond)
+  // the most that a few probed searches up to a time limit take, per limit asked
+  // for so far: nodes, runs of 2^k nodes, discovered and unsettled nodes, nodes
+  // that precede another
+  struct Reach {
+    uint32_t nodes = 0, front = 0, inner = 0;
+    uint32_t pages[10] = {0};
+  };
+  std::map<float, Reach> reach;
+};
+
 // Speed-dependent device edge arrays for one (device, speed).
 struct DevEdges {
   float speed = 0.0f;
@@ -112,6 +128,7 @@ struct DevEdges {
   float min_es_ang = 0.0f;
   float max_w_ang = 0.0f;  // largest route increment (angle + 1e-6 length) of the dual's edges
   std::unique_ptr<AngWaveGraph> ang_wave;
+  std::unique_ptr<DiscGraph> disc;
 };
 
 struct DevGraph {
@@ -289,6 +306,16 @@ struct JobSpec {
   // per-wave records beyond the graph's nodes (land-use dedupe group tables)
   uint32_t extra_records = 0;
 };
+// The jobs' sources with each search in the LDS of one workgroup (cs_disc.hip),
+// in as few launches as their sizes allow; under the graphs' locks. False when
+// none can (nothing ran); what is left over ({job, source position}), having
+// added nothing, goes to rest. cap: settled nodes of a search at most (0: as
+// LDS allows).
+bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, hipStream_t stream, cs_stats &st,
+                 uint32_t *progress, std::vector<uint2> *rest);
+void free_disc(DiscGraph &w);
+void release_disc_workspaces();
+
 // All sources of all jobs in one persistent launch, or only `items`
 // ({job, source position}) when given.
 void launch_shortest_batch(const std::vector<JobSpec> &jobs, uint32_t NT, const Tuning &tune,

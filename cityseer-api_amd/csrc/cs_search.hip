@@ -2080,6 +2080,17 @@ void run_jobs(const std::vector<JobSpec> &specs, uint32_t NT, const Tuning &tune
     p.nbk = std::max(p.nbk, jobs.back().nbk);
     p.maxb = std::max(p.maxb, jobs.back().maxb);
   }
+  std::vector<uint2> left;
+  if constexpr (MODE == kBrandes) {
+    // searches that fit a workgroup's LDS run there; the rest below. (A list of
+    // items is a served slice, whose graph the caller has not locked for the
+    // rows that search keeps with it, or one that has been there already.)
+    if (!explicit_items && launch_disc(specs, NT, tune.cap, stream, st, progress, &left)) {
+      if (left.empty()) return;
+      explicit_items = &left;
+      n_items = left.size();
+    }
+  }
   const uint32_t block = launch_block(tune, p.nbk);
   const uint32_t wpb = block / kWave;
   p.bcap = 1024;
@@ -2474,6 +2485,7 @@ struct ShortestBatch {
 };
 
 void release_search_workspaces() {
+  release_disc_workspaces();
   std::lock_guard<std::mutex> lk(g_ws_mu);
   for (auto &dv : g_ws_pool)
     for (auto &w : dv.second) {

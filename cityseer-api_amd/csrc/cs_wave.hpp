@@ -53,6 +53,18 @@ __device__ __forceinline__ void lds_st(uint32_t *p, uint32_t v) {
 __device__ __forceinline__ uint32_t lds_add(uint32_t *p, uint32_t v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+__device__ __forceinline__ uint32_t lds_min(uint32_t *p, uint32_t v) {
+  return __hip_atomic_fetch_min(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_or(uint32_t *p, uint32_t v) {
+  (void)__hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ uint32_t lds_ld8(const uint8_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_st8(uint8_t *p, uint8_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 // Results shared by all waves (accumulators): device scope.
 __device__ __forceinline__ void gadd_f64(double *p, double v) { unsafeAtomicAdd(p, v); }
 // Orders this wave's earlier memory operations before its later ones (all lanes).

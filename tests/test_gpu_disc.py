@@ -1,0 +1,88 @@
+"""GPU: the LDS shortest search where it could go wrong, against the oracle: exact ties everywhere,
+rows of one to four blocks and beyond, one-way and parallel edges, streets cut into short pieces, a
+single very short edge (nodes that settle alone), either result by itself, more thresholds than one
+variant's registers, source subsets, and searches that outgrow the room the probed sources asked for."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cityseer import _native
+from cityseer.rustalgos.graph import NetworkStructure
+from cityseer.tools import mock
+import oracle.oracle as O
+from oracle.oracle import OracleGraph
+from test_gpu_angular_wave import _grid, _star
+from test_gpu_shortest import SHORTEST_KEYS, assert_close, say, stack
+
+pytestmark = pytest.mark.gpu
+
+
+def _knot():
+    """A lattice at 100 m with one 14 x 14 lattice at 4 m hung on its corner: the searches there reach
+    many times as many nodes as the rest."""
+    a, b = mock.perturbed_lattice(60, seed=5), mock.perturbed_lattice(14, spacing=4.0, jitter=1.0, seed=6)
+    k = len(a.x)
+    return mock.Lattice(x=np.concatenate([a.x, b.x + a.x[0] - 100.0]), y=np.concatenate([a.y, b.y + a.y[0] - 100.0]),
+                        edges=np.concatenate([a.edges, b.edges + k, [[0, k]]]),
+                        length=np.concatenate([a.length, b.length, [np.float32(60.0)]]).astype(np.float32))
+
+
+def _directed(lat, seed):
+    """The lattice with a third of its streets one-way, a tenth doubled and a few loops."""
+    rng = np.random.default_rng(seed)
+    ns = NetworkStructure()
+    n, m = lat.n_nodes, lat.n_edges
+    ns.add_street_nodes_bulk(None, lat.x, lat.y)
+    way = rng.integers(0, 3, m)
+    a = np.concatenate([lat.edges[way != 2, 0], lat.edges[way != 1, 1], lat.edges[:m // 10, 0], [3, 7]])
+    b = np.concatenate([lat.edges[way != 2, 1], lat.edges[way != 1, 0], lat.edges[:m // 10, 1], [3, 7]])
+    length = np.concatenate([lat.length[way != 2], lat.length[way != 1], lat.length[:m // 10] * np.float32(1.00003),
+                             np.float32([30.0, 40.0])])
+    key = np.concatenate([np.zeros(len(a) - m // 10 - 2), np.ones(m // 10), [0, 0]]).astype(np.uint32)
+    ns.add_street_edges_bulk(a, b, key, length)
+    return ns
+
+
+def _short_edge():
+    lat = mock.perturbed_lattice(16, seed=83)
+    lat.length[::37] = np.float32(0.05)
+    return lat
+
+
+@pytest.mark.parametrize("name,distances,kw", [
+    ("grid", [250, 700, 1500], {}),
+    ("star8", [150, 450], {}), ("star16", [300], {}), ("star18", [300], {}),
+    ("pieces", [120, 400, 900], {}),
+    ("directed", [300, 800], {}),
+    ("short edge", [400, 2500], {}),
+    ("five", [200, 300, 400, 500, 3000], {}),
+    ("one", [5000], {}),
+    ("knot", [150, 300], {}),
+    ("five", [350, 800], {"compute_betweenness": False}),
+    ("five", [350, 800], {"compute_closeness": False}),
+    ("five", [600], {"source_indices": [0, 5, 17, 60, 61, 62]}),
+])
+def test_matches_oracle(name, distances, kw):
+    O.set_heap_mode(False)
+    make = {"grid": lambda: _grid(11), "star8": lambda: _star(8, 4, 1.0), "star16": lambda: _star(16, 3, 1.0),
+            "star18": lambda: _star(18, 3, 1.0), "pieces": lambda: mock.decompose_lattice(mock.perturbed_lattice(9, seed=81), 15.0),
+            "short edge": _short_edge, "five": lambda: mock.perturbed_lattice(13, seed=82, diag_frac=0.4),
+            "one": lambda: mock.perturbed_lattice(5, seed=84), "knot": _knot}
+    if name == "directed":
+        ns = _directed(mock.perturbed_lattice(14, seed=85, diag_frac=0.1), 85)
+    else:
+        ns = mock.network_structure_from_lattice(make[name]())
+    say(f"shortest search, {name}: {ns.node_count()} nodes, {distances} m {kw}")
+    res = ns.centrality_shortest(distances=distances, **kw)
+    stats = _native.last_stats()
+    plan = ns._sampling_plan(None, None, None, kw.get("source_indices"))
+    ref, _ = OracleGraph.from_network_structure(ns).centrality_shortest(
+        distances, closeness=kw.get("compute_closeness", True), betweenness=kw.get("compute_betweenness", True),
+        sources=plan["sources"], eligible=plan["eligible"], scale=plan["scale"])
+    got = stack(res, SHORTEST_KEYS, distances)
+    assert np.array_equal(got[0], ref[0])
+    assert_close(got, ref, name)
+    if name == "knot":
+        assert stats["retries"] > 0
