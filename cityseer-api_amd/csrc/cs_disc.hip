@@ -1485,6 +1485,14 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
   return true;
 }
 
+uint32_t disc_nodes(const DevEdges &de, float maxsec) {
+  if (!de.disc) return 0;
+  const auto it = de.disc->reach.find(maxsec);
+  if (it == de.disc->reach.end()) return 0;
+  const uint32_t n = it->second.nodes;
+  return n > kProbeStop ? 4 * 16384u : n + n / 4;
+}
+
 void free_disc(DiscGraph &w) { (void)hipFree(w.row); }
 
 void release_disc_workspaces() {

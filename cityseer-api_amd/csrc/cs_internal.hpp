@@ -313,6 +313,9 @@ struct JobSpec {
 // LDS allows).
 bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, hipStream_t stream, cs_stats &st,
                  uint32_t *progress, std::vector<uint2> *rest);
+// Nodes of a search up to maxsec as far as probed searches tell, with a quarter
+// more (0: none were); under the graph's lock.
+uint32_t disc_nodes(const DevEdges &de, float maxsec);
 void free_disc(DiscGraph &w);
 void release_disc_workspaces();
 

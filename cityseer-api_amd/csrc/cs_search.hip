@@ -2081,7 +2081,9 @@ void run_jobs(const std::vector<JobSpec> &specs, uint32_t NT, const Tuning &tune
     p.maxb = std::max(p.maxb, jobs.back().maxb);
   }
   std::vector<uint2> left;
+  uint32_t cap = 16384u;
   if constexpr (MODE == kBrandes) {
+    const bool probed = !explicit_items;
     // searches that fit a workgroup's LDS run there; the rest below. (A list of
     // items is a served slice, whose graph the caller has not locked for the
     // rows that search keeps with it, or one that has been there already.)
@@ -2090,11 +2092,16 @@ void run_jobs(const std::vector<JobSpec> &specs, uint32_t NT, const Tuning &tune
       explicit_items = &left;
       n_items = left.size();
     }
+    // a source that outgrows its records is searched twice (5,222 sources of a
+    // reach around 16,000, 2,114 of them past it: 19.4 ms): where probed searches
+    // say so, every wave starts with more (14.1 ms)
+    if (probed)
+      for (auto &js : specs) cap = std::max(cap, disc_nodes(*js.de, js.cs.maxsec));
   }
   const uint32_t block = launch_block(tune, p.nbk);
   const uint32_t wpb = block / kWave;
   p.bcap = 1024;
-  p.cap = std::min<uint32_t>({maxN, tune.cap ? tune.cap : 16384u, kSlotLimit});
+  p.cap = std::min<uint32_t>({maxN, tune.cap ? tune.cap : cap, kSlotLimit});
   if (aout && aout->stats) p.st_cap = std::max<uint32_t>(1u, std::min<uint32_t>(aout->n_groups, 4096u));
   const size_t lds = (size_t)wpb * (p.nbk + kWaveLds) * 4;
   const int bpc = std::max(1, blocks_per_cu<MODE>(NT, block, lds));

@@ -86,3 +86,21 @@ def test_matches_oracle(name, distances, kw):
     assert_close(got, ref, name)
     if name == "knot":
         assert stats["retries"] > 0
+
+
+def test_large_reach_is_searched_once():
+    """Too large for a workgroup's LDS and for the usual records of a wave: no source is searched twice."""
+    O.set_heap_mode(False)
+    ns = mock.network_structure_from_lattice(mock.decompose_lattice(mock.perturbed_lattice(46, seed=86), 20.0))
+    n = ns.node_count()
+    src = list(range(0, n, n // 270))
+    say(f"shortest search, large reach: {n} nodes, {len(src)} sources")
+    res = ns.centrality_shortest(distances=[600, 9000], source_indices=src)
+    stats = _native.last_stats()
+    assert stats["nodes_reached"] > 16384 * len(src) and stats["retries"] == 0
+    plan = ns._sampling_plan(None, None, None, src)
+    ref, _ = OracleGraph.from_network_structure(ns).centrality_shortest(
+        [600, 9000], sources=plan["sources"], eligible=plan["eligible"], scale=plan["scale"])
+    got = stack(res, SHORTEST_KEYS, [600, 9000])
+    assert np.array_equal(got[0], ref[0])
+    assert_close(got, ref, "large reach")
