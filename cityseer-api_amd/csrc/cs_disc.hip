@@ -1248,6 +1248,7 @@ static std::vector<DiscClass> disc_plan(const std::vector<JobSpec> &specs, uint3
   hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, specs[0].dg->device), "attribute");
   for (size_t i = 0; i < specs.size(); ++i) {
     const JobSpec &js = specs[i];
+    std::lock_guard<std::mutex> lk(js.de->disc_mu);
     if (!js.n_sources || !disc_takes(js, tmp, stream)) continue;
     DiscGraph &w = *js.de->disc;
     DiscArgs a;
@@ -1400,7 +1401,6 @@ static void disc_enqueue(const DiscClass &d, uint32_t blocks, char *ctl, hipStre
   else if (d.NT <= 2) hipLaunchKernelGGL(k_disc<2>, grid, block, d.lds, stream, d.a);
   else if (d.NT <= 4) hipLaunchKernelGGL(k_disc<4>, grid, block, d.lds, stream, d.a);
   else hipLaunchKernelGGL(k_disc<8>, grid, block, d.lds, stream, d.a);
-  hip_check(hipGetLastError(), "k_disc launch");
 }
 
 bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, hipStream_t stream, cs_stats &st,
@@ -1444,6 +1444,7 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
     disc_args(d, ctl, fail_list, items, jobs, scratch, progress, blocks);
     hip_check(hipEventRecord(ws->e0, stream), "event");
     disc_enqueue(d, blocks, ctl, stream);
+    hip_check(hipGetLastError(), "k_disc launch");
     hip_check(hipEventRecord(ws->e1, stream), "event");
     uint32_t h[64];
     hip_check(hipMemcpyAsync(h, ctl, 256, hipMemcpyDeviceToHost, stream), "copy");
@@ -1485,7 +1486,109 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
   return true;
 }
 
+// The launches of a fixed set of jobs, for a batch that replays them from a
+// graph: memory of their own, nothing of it changed between runs.
+struct DiscBatch {
+  struct Part {
+    DiscClass d;
+    uint32_t blocks = 0;
+    char *ctl = nullptr;
+    uint32_t *fail = nullptr;
+  };
+  std::vector<Part> parts;
+  std::vector<void *> bufs;
+  char *ctl = nullptr;  // [parts][256]
+  uint32_t waves = 0;
+  ~DiscBatch() {
+    for (void *q : bufs) (void)hipFree(q);
+  }
+  void *mem(size_t bytes) {
+    void *q = nullptr;
+    hip_check(hipMalloc(&q, std::max<size_t>(bytes, 1)), "hipMalloc batch");
+    bufs.push_back(q);
+    return q;
+  }
+};
+
+DiscBatch *disc_batch_new(const std::vector<JobSpec> &specs, uint32_t NT, int device, hipStream_t stream,
+                          std::vector<uint2> *rest) {
+  auto b = std::make_unique<DiscBatch>();
+  DevVec tmp;
+  struct Release {
+    DevVec &v;
+    ~Release() { v.release(); }
+  } release{tmp};
+  std::vector<DiscClass> work = disc_plan(specs, NT, 0, tmp, stream, rest);
+  size_t scratch = 0;
+  for (DiscClass &c : work) {
+    DiscBatch::Part p;
+    p.d = std::move(c);
+    if (!disc_shape(p.d, 0, device, true, &p.blocks)) {
+      for (uint32_t i = 0; i < p.d.n; ++i) {
+        const uint2 x = p.d.items.empty() ? make_uint2(0u, i) : p.d.items[i];
+        rest->push_back(make_uint2(p.d.which[x.x], x.y));
+      }
+      continue;
+    }
+    size_t free_b = 0, total_b = 0;
+    hip_check(hipMemGetInfo(&free_b, &total_b), "meminfo");
+    p.blocks = (uint32_t)std::min<size_t>(p.blocks, std::max<size_t>(1, free_b / 4 / p.d.a.stride));
+    scratch = std::max(scratch, p.d.a.stride * p.blocks);
+    b->waves = std::max(b->waves, p.blocks * p.d.waves);
+    b->parts.push_back(std::move(p));
+  }
+  if (b->parts.empty()) return nullptr;
+  char *ws = static_cast<char *>(b->mem(scratch));  // (the launches follow one another)
+  b->ctl = static_cast<char *>(b->mem(256 * b->parts.size()));
+  for (size_t i = 0; i < b->parts.size(); ++i) {
+    DiscBatch::Part &p = b->parts[i];
+    p.ctl = b->ctl + 256 * i;
+    p.fail = static_cast<uint32_t *>(b->mem(4ull * p.d.n));
+    DiscJob *jobs = static_cast<DiscJob *>(b->mem(sizeof(DiscJob) * p.d.jobs.size()));
+    hip_check(hipMemcpy(jobs, p.d.jobs.data(), sizeof(DiscJob) * p.d.jobs.size(), hipMemcpyHostToDevice), "copy");
+    uint2 *items = nullptr;
+    if (!p.d.items.empty()) {
+      items = static_cast<uint2 *>(b->mem(sizeof(uint2) * p.d.n));
+      hip_check(hipMemcpy(items, p.d.items.data(), sizeof(uint2) * p.d.n, hipMemcpyHostToDevice), "copy");
+    }
+    disc_args(p.d, p.ctl, p.fail, items, jobs, ws, nullptr, p.blocks);
+  }
+  return b.release();
+}
+
+void disc_batch_delete(DiscBatch *b) { delete b; }
+
+void disc_batch_enqueue(const DiscBatch &b, hipStream_t stream) {
+  for (const DiscBatch::Part &p : b.parts) disc_enqueue(p.d, p.blocks, p.ctl, stream);
+}
+
+void disc_batch_collect(const DiscBatch &b, hipStream_t stream, cs_stats &st, std::vector<uint2> *retry) {
+  std::vector<uint32_t> h(64 * b.parts.size());
+  hip_check(hipMemcpyAsync(h.data(), b.ctl, 4 * h.size(), hipMemcpyDeviceToHost, stream), "copy");
+  hip_check(hipStreamSynchronize(stream), "sync");
+  st.waves = std::max(st.waves, b.waves);
+  for (size_t i = 0; i < b.parts.size(); ++i) {
+    const DiscBatch::Part &p = b.parts[i];
+    const uint32_t *c = &h[64 * i];
+    unsigned long long stv[4];
+    std::memcpy(stv, c + 32, 32);
+    st.nodes_reached += stv[0];
+    st.edges_scanned += stv[1];
+    st.within_sum += stv[2];
+    const uint32_t n_failed = c[kXcd];
+    if (!n_failed) continue;
+    if (c[kXcd + 1] & kFailInternal) fail(CS_EINTERNAL, "search invariant violated (settle order)");
+    std::vector<uint32_t> fl(n_failed);
+    hip_check(hipMemcpy(fl.data(), p.fail, 4ull * n_failed, hipMemcpyDeviceToHost), "copy");
+    for (uint32_t k : fl) {
+      const uint2 x = p.d.items.empty() ? make_uint2(0u, k) : p.d.items[k];
+      retry->push_back(make_uint2(p.d.which[x.x], x.y));
+    }
+  }
+}
+
 uint32_t disc_nodes(const DevEdges &de, float maxsec) {
+  std::lock_guard<std::mutex> lk(de.disc_mu);
   if (!de.disc) return 0;
   const auto it = de.disc->reach.find(maxsec);
   if (it == de.disc->reach.end()) return 0;

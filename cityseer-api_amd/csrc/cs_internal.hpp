@@ -129,6 +129,7 @@ struct DevEdges {
   float max_w_ang = 0.0f;  // largest route increment (angle + 1e-6 length) of the dual's edges
   std::unique_ptr<AngWaveGraph> ang_wave;
   std::unique_ptr<DiscGraph> disc;
+  mutable std::mutex disc_mu;  // its building and its table of probed searches
 };
 
 struct DevGraph {
@@ -307,14 +308,23 @@ struct JobSpec {
   uint32_t extra_records = 0;
 };
 // The jobs' sources with each search in the LDS of one workgroup (cs_disc.hip),
-// in as few launches as their sizes allow; under the graphs' locks. False when
-// none can (nothing ran); what is left over ({job, source position}), having
+// in as few launches as their sizes allow. False when none can (nothing ran);
+// what is left over ({job, source position}), having
 // added nothing, goes to rest. cap: settled nodes of a search at most (0: as
 // LDS allows).
 bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, hipStream_t stream, cs_stats &st,
                  uint32_t *progress, std::vector<uint2> *rest);
+// The same for a fixed set of jobs run many times: prepared once (null: none
+// can), enqueued (under capture too), and its counts and the items that ran out
+// of room taken after each run.
+struct DiscBatch;
+DiscBatch *disc_batch_new(const std::vector<JobSpec> &specs, uint32_t NT, int device, hipStream_t stream,
+                          std::vector<uint2> *rest);
+void disc_batch_delete(DiscBatch *b);
+void disc_batch_enqueue(const DiscBatch &b, hipStream_t stream);
+void disc_batch_collect(const DiscBatch &b, hipStream_t stream, cs_stats &st, std::vector<uint2> *retry);
 // Nodes of a search up to maxsec as far as probed searches tell, with a quarter
-// more (0: none were); under the graph's lock.
+// more (0: none were).
 uint32_t disc_nodes(const DevEdges &de, float maxsec);
 void free_disc(DiscGraph &w);
 void release_disc_workspaces();

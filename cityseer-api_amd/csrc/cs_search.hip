@@ -2268,7 +2268,8 @@ struct ShortestBatch {
   int device = 0;
   Tuning tune;
   bool ready = false;
-  uint64_t n_items = 0;
+  uint64_t n_items = 0;       // of the search in scratch
+  DiscBatch *disc = nullptr;  // the others
   Plan p{};
   uint32_t block = kBlock, wpb = kBlock / kWave, waves = 0;
   size_t lds = 0;
@@ -2295,6 +2296,8 @@ struct ShortestBatch {
     d_items = nullptr;
     d_ctl = d_fail = nullptr;
     d_stats = nullptr;
+    disc_batch_delete(disc);
+    disc = nullptr;
     ws.release();
     ready = false;
   }
@@ -2317,10 +2320,17 @@ struct ShortestBatch {
       p.nbk = std::max(p.nbk, jobs.back().nbk);
       p.maxb = std::max(p.maxb, jobs.back().maxb);
     }
+    // searches that fit a workgroup's LDS run there (8 towns, 39,475 sources at
+    // 1,600 m: 3.95 -> 3.00 ms); the rest below, as all with a slot capacity asked for
+    items.clear();
+    if (!tune.cap) disc = disc_batch_new(specs, NT, device, stream, &items);
+    if (disc) n_items = items.size();
+    uint32_t cap = 16384u;
+    for (auto &js : specs) cap = std::max(cap, disc_nodes(*js.de, js.cs.maxsec));
     block = launch_block(tune, p.nbk);
     wpb = block / kWave;
     p.bcap = 1024;
-    p.cap = std::min<uint32_t>({maxN, tune.cap ? tune.cap : 16384u, kSlotLimit});
+    p.cap = std::min<uint32_t>({maxN, tune.cap ? tune.cap : cap, kSlotLimit});
     lds = (size_t)wpb * (p.nbk + kWaveLds) * 4;
     const DevInfo &di = dev_info(device);
     const int bpc = std::max(1, blocks_per_cu<kBrandes>(NT, block, lds));
@@ -2330,11 +2340,11 @@ struct ShortestBatch {
     size_t free_b = 0, total_b = 0;
     hip_check(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
     const uint32_t by_mem = (uint32_t)std::min<size_t>((free_b / 4) / (p.stride + kRecBytes * maxN), 1u << 20);
-    if (by_mem < wpb) fail(CS_ENOMEM, "batch too large for the search workspace on this device");
+    if (n_items && by_mem < wpb) fail(CS_ENOMEM, "batch too large for the search workspace on this device");
     waves = std::min<uint32_t>((uint32_t)std::min<uint64_t>(n_items, resident), by_mem);
     waves = std::max<uint32_t>(wpb, (waves + wpb - 1) / wpb * wpb);
-    items.clear();
-    if (specs.size() > 1) {
+    if (!disc) items.clear();
+    if (!disc && specs.size() > 1) {
       items.reserve(n_items);
       for (uint32_t jb = 0; jb < specs.size(); ++jb)
         for (uint32_t i = 0; i < specs[jb].n_sources; ++i) items.push_back(make_uint2(jb, i));
@@ -2348,7 +2358,7 @@ struct ShortestBatch {
     hip_check(hipMalloc(&d_stats, 32), "hipMalloc stats");
     hip_check(hipMalloc(&d_fail, 4 * std::max<uint64_t>(n_items, 1)), "hipMalloc fail");
     ws.device = device;
-    prepare_ws(ws, maxN, p.stride, waves, 0, stream);
+    if (n_items) prepare_ws(ws, maxN, p.stride, waves, 0, stream);
     hip_check(hipStreamSynchronize(stream), "sync");
     // capture: clear control words, statistics and accumulators, then search
     SearchArgs a = args();
@@ -2359,7 +2369,8 @@ struct ShortestBatch {
       const size_t grid = std::min<size_t>((z.words + 255) / 256, 4096);
       if (z.words) hipLaunchKernelGGL(k_zero64, dim3((uint32_t)grid), dim3(256), 0, stream, z.ptr, z.words);
     }
-    launch_nt<kBrandes>(NT, waves / wpb, block, lds, stream, a);
+    if (disc) disc_batch_enqueue(*disc, stream);
+    if (n_items) launch_nt<kBrandes>(NT, waves / wpb, block, lds, stream, a);
     hipError_t le = hipGetLastError();
     hipError_t ce = hipStreamEndCapture(stream, &graph);
     hip_check(le, "k_search capture");
@@ -2404,7 +2415,7 @@ struct ShortestBatch {
 
   void run(hipStream_t stream, cs_stats &st) {
     if (!ready) prepare(stream);
-    if (n_items == 0) return;
+    if (n_items == 0 && !disc) return;
     // epochs: every wave may use up to n_items of them per run
     if (ws.epoch_hi + n_items + 2 >= 0xfffffff0ull) {
       hip_check(hipMemsetAsync(ws.keys, 0, kRecBytes * ws.ncap * ws.key_waves, stream), "hipMemset keys");
@@ -2428,23 +2439,26 @@ struct ShortestBatch {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     st.kernel_ms += ms;
-    st.waves = waves;
+    st.waves = n_items ? waves : 0;
     st.nodes_reached += stv[0];
     st.edges_scanned += stv[1];
     st.within_sum += stv[2];
+    std::vector<uint2> retry;
+    if (disc) disc_batch_collect(*disc, stream, st, &retry);
     const uint32_t n_failed = ctl[kXcd], flags = ctl[kXcd + 1];
-    if (n_failed == 0) return;
+    if (n_failed == 0 && retry.empty()) return;
     if (flags & kFailWide) fail_wide_row();
     if (flags & kFailInternal) fail(CS_EINTERNAL, "search invariant violated (bucket order)");
     if (flags & kFailRing) fail(CS_EINTERNAL, "bucket ring window exceeded");
-    st.retries += n_failed;
-    std::vector<uint32_t> fl(n_failed);
-    hip_check(hipMemcpy(fl.data(), d_fail, 4ull * n_failed, hipMemcpyDeviceToHost), "copy");
-    std::vector<uint2> retry(n_failed);
-    for (uint32_t i = 0; i < n_failed; ++i) retry[i] = items.empty() ? make_uint2(0u, fl[i]) : items[fl[i]];
+    st.retries += n_failed + (uint32_t)retry.size();
     Tuning t2 = tune;
-    if (p.cap >= kSlotLimit) fail(CS_EINVAL, "a source reaches more than 4,194,304 nodes, the search's slot limit");
-    t2.cap = std::min<uint32_t>(std::max<uint32_t>(p.cap * 4, 4096), kSlotLimit);
+    if (n_failed) {
+      std::vector<uint32_t> fl(n_failed);
+      hip_check(hipMemcpy(fl.data(), d_fail, 4ull * n_failed, hipMemcpyDeviceToHost), "copy");
+      for (uint32_t k : fl) retry.push_back(items.empty() ? make_uint2(0u, k) : items[k]);
+      if (p.cap >= kSlotLimit) fail(CS_EINVAL, "a source reaches more than 4,194,304 nodes, the search's slot limit");
+      t2.cap = std::min<uint32_t>(std::max<uint32_t>(p.cap * 4, 4096), kSlotLimit);
+    }
     run_jobs<kBrandes>(specs, NT, t2, nullptr, stream, st, &retry);
   }
 

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from cityseer import _native
+from cityseer.batch import CentralityBatch
 from cityseer.rustalgos.graph import NetworkStructure
 from cityseer.tools import mock
 import oracle.oracle as O
@@ -104,3 +105,23 @@ def test_large_reach_is_searched_once():
     got = stack(res, SHORTEST_KEYS, [600, 9000])
     assert np.array_equal(got[0], ref[0])
     assert_close(got, ref, "large reach")
+
+
+def test_batch_mixes_searches_and_replays():
+    """One batch of searches in LDS, of two sizes, some out of room, and in scratch; every replay the same."""
+    nets = [mock.network_structure_from_lattice(x) for x in
+            (_knot(), _star(18, 3, 1.0), mock.perturbed_lattice(13, seed=82), mock.perturbed_lattice(50, seed=87))]
+    asked = [[150, 300], [300], [200, 500], [2500]]
+    alone = [stack(ns.centrality_shortest(distances=d), SHORTEST_KEYS, d) for ns, d in zip(nets, asked)]
+    with CentralityBatch() as batch:
+        for ns, d in zip(nets, asked):
+            batch.add_shortest(ns, distances=d)
+        for k in range(3):
+            say(f"batch of {len(nets)} networks, run {k}")
+            stats = batch.run()
+            assert stats["retries"] > 0
+            for i, (res, d) in enumerate(zip(batch.results(), asked)):
+                got = stack(res, SHORTEST_KEYS, d)
+                assert np.array_equal(got[0], alone[i][0])
+                assert_close(got, alone[i], f"network {i}, run {k}")
+            nets[2].centrality_shortest(distances=[400])
