@@ -1416,7 +1416,7 @@ void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<u
     a.n_fail = d_ctl + 1;
     a.fail_flags = d_ctl + 2;
     a.fail_list = d_fail;
-    a.progress = lanes <= kProgressSlots ? progress : nullptr;
+    a.progress = progress_room(progress, lanes);
     hip_check(hipEventRecord(e0, stream), "event");
     if (p.bq_cap)
       hipLaunchKernelGGL(k_angular<1>, dim3(lanes / kBlock), dim3(kBlock), 0, stream, a);

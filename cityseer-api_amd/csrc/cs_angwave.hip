@@ -1335,7 +1335,7 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
     a.fail_list = d_fail;
     a.stats = reinterpret_cast<unsigned long long *>(ctl + 128);
     for (uint32_t x = 0; x <= kXcd; ++x) a.xbeg[x] = (uint32_t)((uint64_t)n_list * x / kXcd);
-    a.progress = waves <= kProgressSlots ? progress : nullptr;
+    a.progress = progress_room(progress, waves);
     hip_check(hipMemsetAsync(ctl, 0, 64, stream), "memset ctl");
     hip_check(hipEventRecord(ws.e0, stream), "event");
     hipLaunchKernelGGL(k_angular_wave, dim3(waves), dim3(kWave), lds, stream, a);

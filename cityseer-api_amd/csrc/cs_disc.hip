@@ -1391,7 +1391,7 @@ static void disc_args(DiscClass &d, char *ctl, uint32_t *fail, const uint2 *item
   a.fail_flags = a.next + kXcd + 1;
   a.fail_list = fail;
   for (uint32_t x = 0; x <= kXcd; ++x) a.xbeg[x] = (uint32_t)((uint64_t)d.n * x / kXcd);
-  a.progress = blocks <= kProgressSlots ? progress : nullptr;
+  a.progress = progress_room(progress, blocks);
 }
 
 static void disc_enqueue(const DiscClass &d, uint32_t blocks, char *ctl, hipStream_t stream) {

@@ -239,6 +239,21 @@ void set_node_order_from_xy(Graph &g, const double *x, const double *y) {
 // kernels write them through the device's view of host memory.
 std::mutex g_progress_mu;
 std::vector<std::pair<uint32_t *, uint32_t *>> g_progress_pool;  // {host, device}
+std::map<const uint32_t *, uint32_t> g_progress_used;  // by device address: counts the last call's launches may have written
+
+uint32_t progress_used(const uint32_t *dev) {
+  std::lock_guard<std::mutex> lk(g_progress_mu);
+  const auto it = g_progress_used.find(dev);
+  return it == g_progress_used.end() ? kProgressSlots : it->second;
+}
+
+uint32_t *progress_room(uint32_t *progress, uint32_t n) {
+  if (!progress || n > kProgressSlots) return nullptr;
+  std::lock_guard<std::mutex> lk(g_progress_mu);
+  uint32_t &used = g_progress_used[progress];
+  used = std::max(used, n);
+  return progress;
+}
 
 uint32_t *progress_begin(Graph &g, uint64_t settled_on_host) {
   uint32_t *slots = g.progress_slots.load(std::memory_order_acquire);
@@ -262,7 +277,11 @@ uint32_t *progress_begin(Graph &g, uint64_t settled_on_host) {
     slots = pr.first;
   }
   g.progress_host.store(settled_on_host, std::memory_order_relaxed);
-  for (uint32_t i = 0; i < kProgressSlots; ++i) __atomic_store_n(&slots[i], 0u, __ATOMIC_RELAXED);
+  for (uint32_t i = 0, n = progress_used(g.progress_dev); i < n; ++i) __atomic_store_n(&slots[i], 0u, __ATOMIC_RELAXED);
+  {
+    std::lock_guard<std::mutex> lk(g_progress_mu);
+    g_progress_used[g.progress_dev] = 0;
+  }
   g.progress_slots.store(slots, std::memory_order_release);
   return g.progress_dev;
 }
@@ -270,7 +289,7 @@ uint32_t *progress_begin(Graph &g, uint64_t settled_on_host) {
 void progress_finish(Graph &g, uint64_t n) {
   uint64_t counted = 0;
   if (const uint32_t *slots = g.progress_slots.load(std::memory_order_acquire))
-    for (uint32_t i = 0; i < kProgressSlots; ++i) counted += __atomic_load_n(&slots[i], __ATOMIC_RELAXED);
+    for (uint32_t i = 0, k = progress_used(g.progress_dev); i < k; ++i) counted += __atomic_load_n(&slots[i], __ATOMIC_RELAXED);
   g.progress_host.store(n > counted ? n - counted : 0, std::memory_order_relaxed);
 }
 
@@ -464,6 +483,121 @@ struct DevBuf {
   }
 };
 
+// Device buffers and streams kept between calls: a call took up to ten
+// allocations, and each free waits for the device (64 sources, with the stream and
+// the progress counts 300 -> 191 us a call). Handed on only when the call has waited for its stream; one that ends in
+// an error frees its own.
+struct Kept {
+  std::mutex mu;
+  struct Buf {
+    int dev;
+    void *p;
+    size_t bytes;
+  };
+  std::vector<Buf> bufs;
+  size_t total = 0;
+  std::vector<std::pair<int, hipStream_t>> streams;
+  static constexpr size_t kMost = 256u << 20, kMostBufs = 64, kMostStreams = 16;
+
+  void release() {
+    std::lock_guard<std::mutex> lk(mu);
+    for (Buf &b : bufs) (void)hipFree(b.p);
+    for (auto &x : streams) (void)hipStreamDestroy(x.second);
+    bufs.clear();
+    streams.clear();
+    total = 0;
+  }
+};
+Kept &kept() {
+  static Kept *k = new Kept;  // (outlives the runtime's own teardown)
+  return *k;
+}
+
+struct KeptBuf {
+  void *p = nullptr;
+  size_t bytes = 0;
+  int dev = 0, errors = std::uncaught_exceptions();
+  explicit KeptBuf(size_t need) {
+    need = std::max<size_t>(need, 256);
+    dev = current_device();
+    Kept &k = kept();
+    {
+      std::lock_guard<std::mutex> lk(k.mu);
+      size_t best = k.bufs.size();
+      for (size_t i = 0; i < k.bufs.size(); ++i) {
+        const Kept::Buf &b = k.bufs[i];
+        if (b.dev == dev && b.bytes >= need && b.bytes / 2 <= need + 32768 &&
+            (best == k.bufs.size() || b.bytes < k.bufs[best].bytes))
+          best = i;
+      }
+      if (best < k.bufs.size()) {
+        p = k.bufs[best].p;
+        bytes = k.bufs[best].bytes;
+        k.total -= bytes;
+        k.bufs[best] = k.bufs.back();
+        k.bufs.pop_back();
+      }
+    }
+    if (p) return;
+    bytes = (need + 4095) & ~(size_t)4095;
+    if (hipMalloc(&p, bytes) == hipSuccess) return;
+    (void)hipGetLastError();
+    p = nullptr;
+    k.release();
+    hip_check(hipMalloc(&p, bytes), "hipMalloc");
+  }
+  ~KeptBuf() {
+    if (!p) return;
+    Kept &k = kept();
+    if (std::uncaught_exceptions() <= errors) {
+      std::lock_guard<std::mutex> lk(k.mu);
+      if (k.total + bytes <= Kept::kMost && k.bufs.size() < Kept::kMostBufs) {
+        k.bufs.push_back({dev, p, bytes});
+        k.total += bytes;
+        return;
+      }
+    }
+    (void)hipFree(p);
+  }
+  KeptBuf(const KeptBuf &) = delete;
+  KeptBuf &operator=(const KeptBuf &) = delete;
+  template <typename T>
+  T *as() const {
+    return static_cast<T *>(p);
+  }
+};
+
+struct KeptStream {
+  hipStream_t s = nullptr;
+  int dev = 0, errors = std::uncaught_exceptions();
+  KeptStream() {
+    dev = current_device();
+    Kept &k = kept();
+    std::lock_guard<std::mutex> lk(k.mu);
+    for (size_t i = 0; i < k.streams.size() && !s; ++i)
+      if (k.streams[i].first == dev) {
+        s = k.streams[i].second;
+        k.streams[i] = k.streams.back();
+        k.streams.pop_back();
+      }
+    if (!s) hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "stream");
+  }
+  ~KeptStream() {
+    Kept &k = kept();
+    if (std::uncaught_exceptions() <= errors) {
+      std::lock_guard<std::mutex> lk(k.mu);
+      if (k.streams.size() < Kept::kMostStreams) {
+        k.streams.emplace_back(dev, s);
+        return;
+      }
+    }
+    (void)hipStreamDestroy(s);
+  }
+  KeptStream(const KeptStream &) = delete;
+  KeptStream &operator=(const KeptStream &) = delete;
+  operator hipStream_t() const { return s; }
+};
+
 void check_params(const Graph &g, const cs_params *p) {
   if (!p) fail(CS_EINVAL, "params must not be NULL");
   if (p->n_thresholds == 0) fail(CS_EINVAL, "at least one distance threshold is required");
@@ -570,11 +704,6 @@ void unpack_acc_strided(const double *acc, uint32_t N, uint32_t M, uint32_t T, u
         for (uint32_t d = 0; d < N; ++d) dst[iperm[d]] = src[d];
       }
     }
-}
-
-void unpack_acc(const std::vector<double> &acc, uint32_t N, uint32_t M, uint32_t T, double *out,
-                const uint32_t *iperm) {
-  unpack_acc_strided(acc.data(), N, M, T, T, out, iperm);
 }
 
 void scale_rows(double *out, uint32_t N, uint32_t T, uint32_t m0, uint32_t m1, double s, uint32_t t0,
@@ -836,7 +965,7 @@ uint64_t cs_graph_progress(const cs_graph *h) {
   const Graph &g = h->g;
   uint64_t n = g.progress_host.load(std::memory_order_relaxed);
   if (const uint32_t *slots = g.progress_slots.load(std::memory_order_acquire))
-    for (uint32_t i = 0; i < kProgressSlots; ++i) n += __atomic_load_n(&slots[i], __ATOMIC_RELAXED);
+    for (uint32_t i = 0, k = progress_used(g.progress_dev); i < k; ++i) n += __atomic_load_n(&slots[i], __ATOMIC_RELAXED);
   return n;
 }
 
@@ -859,8 +988,8 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
     to_device_sources(g, ss);
     const std::vector<uint8_t> elig = to_device_u8(g, p->eligible);
     const uint32_t N = g.n, T = p->n_thresholds, M = 7;
-    OwnedStream stream;
-    DevBuf acc(sizeof(double) * (size_t)N * M * T), reach(4 * T), d_src(4 * ss.src.size()),
+    KeptStream stream;
+    KeptBuf acc(sizeof(double) * (size_t)N * M * T), reach(4 * T), d_src(4 * ss.src.size()),
         d_wt(4 * ss.src.size()), d_cyc(4 * ss.src.size()), d_elig(N);
     hip_check(hipMemsetAsync(acc.p, 0, sizeof(double) * (size_t)N * M * T, stream), "memset");
     hip_check(hipMemsetAsync(reach.p, 0, 4 * T, stream), "memset");
@@ -870,10 +999,12 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
       hip_check(hipMemcpyAsync(d_cyc.p, ss.cyc.data(), 4 * ss.cyc.size(), hipMemcpyHostToDevice, stream), "copy");
     }
     hip_check(hipMemcpyAsync(d_elig.p, elig.data(), N, hipMemcpyHostToDevice, stream), "copy");
+    const uint32_t *d_perm = nullptr;
     {
       std::lock_guard<std::mutex> lk(g.mu);
       DevGraph &dg = device_graph(g, dev);
       DevEdges &de = device_edges(g, dg, spec.speed);
+      if (!g.identity_order) d_perm = dg.perm;
       run_shortest_checks(g, p);
       uint32_t *prog = progress_begin(g, p->n_sources - ss.src.size());
       // a call of several threshold chunks reports progress in its last one
@@ -884,14 +1015,12 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
                         t0 + kMaxT >= T ? prog : nullptr);
       progress_finish(g, p->n_sources);
     }
-    std::vector<double> hacc((size_t)N * M * T);
     std::vector<uint32_t> hreach(T);
-    hip_check(hipMemcpyAsync(hacc.data(), acc.p, sizeof(double) * hacc.size(), hipMemcpyDeviceToHost, stream),
-              "copy out");
+    KeptBuf tmp(sizeof(double) * (size_t)N * M * T);
+    results_out(acc.as<double>(), N, M, T, T, d_perm, 5, 6, p->compute_betweenness ? p->betw_scale : 1.0, tmp.as<double>(), out,
+                stream);
     hip_check(hipMemcpyAsync(hreach.data(), reach.p, 4 * T, hipMemcpyDeviceToHost, stream), "copy out");
     hip_check(hipStreamSynchronize(stream), "sync");
-    unpack_acc(hacc, N, M, T, out, result_order(g));
-    if (p->compute_betweenness) scale_rows(out, N, T, 5, 6, p->betw_scale);
     if (reach_totals)
       for (uint32_t i = 0; i < T; ++i) reach_totals[i] = hreach[i];
     t_stats.sources = ss.src.size();
@@ -1002,13 +1131,14 @@ int cs_betweenness_od_shortest(cs_graph *h, const cs_params *p, uint32_t n_pairs
     const uint32_t T = p->n_thresholds, M = 7;
     const uint32_t ns = (uint32_t)src.size();
     const int dev = current_device();
-    OwnedStream stream;
-    DevBuf acc(sizeof(double) * (size_t)N * M * T), d_src(4 * std::max<size_t>(ns, 1)),
+    KeptStream stream;
+    KeptBuf acc(sizeof(double) * (size_t)N * M * T), d_src(4 * std::max<size_t>(ns, 1)),
         d_wt(4 * std::max<size_t>(ns, 1)), d_elig(N), d_off(4 * off.size()), d_dest(4 * std::max<size_t>(dest.size(), 1)),
         d_w(4 * std::max<size_t>(w.size(), 1));
     const std::vector<float> ones(std::max<size_t>(ns, 1), 1.0f);
     hip_check(hipMemsetAsync(acc.p, 0, sizeof(double) * (size_t)N * M * T, stream), "memset");
     hip_check(hipMemsetAsync(d_elig.p, 0, N, stream), "memset");
+    const uint32_t *d_perm = nullptr;
     if (ns) {
       hip_check(hipMemcpyAsync(d_src.p, src.data(), 4 * ns, hipMemcpyHostToDevice, stream), "copy");
       hip_check(hipMemcpyAsync(d_wt.p, ones.data(), 4 * ns, hipMemcpyHostToDevice, stream), "copy");
@@ -1018,6 +1148,7 @@ int cs_betweenness_od_shortest(cs_graph *h, const cs_params *p, uint32_t n_pairs
       std::lock_guard<std::mutex> lk(g.mu);
       DevGraph &dg = device_graph(g, dev);
       DevEdges &de = device_edges(g, dg, p->speed_m_s);
+      if (!g.identity_order) d_perm = dg.perm;
       check_betweenness_graph(g);
       uint32_t *prog = progress_begin(g, N - ns);
       for (uint32_t t0 = 0; t0 < T; t0 += kMaxT) {
@@ -1035,12 +1166,9 @@ int cs_betweenness_od_shortest(cs_graph *h, const cs_params *p, uint32_t n_pairs
                               t0 + kMaxT >= T ? prog : nullptr);
       }
     }
-    std::vector<double> hacc((size_t)N * M * T);
-    hip_check(hipMemcpyAsync(hacc.data(), acc.p, sizeof(double) * hacc.size(), hipMemcpyDeviceToHost, stream),
-              "copy out");
+    // rows 5 and 6 (betweenness, betweenness_beta) of the [M][T][N] accumulators, by way of the others
+    results_out(acc.as<double>() + (size_t)5 * T * N, N, 2, T, T, d_perm, 0, 0, 1.0, acc.as<double>(), out, stream);
     hip_check(hipStreamSynchronize(stream), "sync");
-    // rows 5 and 6 (betweenness, betweenness_beta) of the [M][T][N] accumulators
-    unpack_acc_strided(hacc.data() + (size_t)5 * T * N, N, 2, T, T, out, result_order(g));
     t_stats.sources = ns;
     progress_finish(g, N);
   });
@@ -1070,8 +1198,8 @@ int cs_segment_centrality(cs_graph *h, const cs_params *p, double *out) {
     std::lock_guard<std::mutex> lk(g.mu);
     DevGraph &dg = device_graph(g, dev);
     DevEdges &de = device_edges(g, dg, p->speed_m_s);
-    OwnedStream stream;
-    DevBuf acc(sizeof(double) * (size_t)N * M * T), d_src(4 * srcs.size());
+    KeptStream stream;
+    KeptBuf acc(sizeof(double) * (size_t)N * M * T), d_src(4 * srcs.size());
     hip_check(hipMemsetAsync(acc.p, 0, sizeof(double) * (size_t)N * M * T, stream), "memset");
     if (!srcs.empty())
       hip_check(hipMemcpyAsync(d_src.p, srcs.data(), 4 * srcs.size(), hipMemcpyHostToDevice, stream), "copy");
@@ -1079,11 +1207,9 @@ int cs_segment_centrality(cs_graph *h, const cs_params *p, double *out) {
     for (uint32_t t0 = 0; t0 < T; t0 += kMaxT)
       launch_segment(g, dg, de, make_spec(p, t0, chunk_len(T, t0)), d_src.as<uint32_t>(), (uint32_t)srcs.size(),
                      acc.as<double>() + (size_t)t0 * N, stream, t_stats, T, t0 + kMaxT >= T ? prog : nullptr);
-    std::vector<double> hacc((size_t)N * M * T);
-    hip_check(hipMemcpyAsync(hacc.data(), acc.p, sizeof(double) * hacc.size(), hipMemcpyDeviceToHost, stream),
-              "copy out");
+    KeptBuf tmp(sizeof(double) * (size_t)N * M * T);
+    results_out(acc.as<double>(), N, M, T, T, g.identity_order ? nullptr : dg.perm, 0, 0, 1.0, tmp.as<double>(), out, stream);
     hip_check(hipStreamSynchronize(stream), "sync");
-    unpack_acc(hacc, N, M, T, out, result_order(g));
     t_stats.sources = srcs.size();
     progress_finish(g, p->n_sources);
   });
@@ -1105,8 +1231,8 @@ int cs_centrality_simplest(cs_graph *h, const cs_params *p, double *out, uint32_
     std::lock_guard<std::mutex> lk(g.mu);
     DevGraph &dg = device_graph(g, dev);
     DevEdges &de = device_edges(g, dg, p->speed_m_s);
-    OwnedStream stream;
-    DevBuf acc(sizeof(double) * (size_t)N * M * T), reach(4 * T), d_src(4 * ss.src.size()),
+    KeptStream stream;
+    KeptBuf acc(sizeof(double) * (size_t)N * M * T), reach(4 * T), d_src(4 * ss.src.size()),
         d_wt(4 * ss.src.size()), d_elig(N);
     hip_check(hipMemsetAsync(acc.p, 0, sizeof(double) * (size_t)N * M * T, stream), "memset");
     hip_check(hipMemsetAsync(reach.p, 0, 4 * T, stream), "memset");
@@ -1120,14 +1246,12 @@ int cs_centrality_simplest(cs_graph *h, const cs_params *p, double *out, uint32_
       launch_simplest(g, dg, de, make_spec(p, t0, chunk_len(T, t0)), d_src.as<uint32_t>(), d_wt.as<float>(),
                       (uint32_t)ss.src.size(), d_elig.as<uint8_t>(), acc.as<double>() + (size_t)t0 * N,
                       reach.as<uint32_t>() + t0, stream, t_stats, T, t0 + kMaxT >= T ? prog : nullptr);
-    std::vector<double> hacc((size_t)N * M * T);
     std::vector<uint32_t> hreach(T);
-    hip_check(hipMemcpyAsync(hacc.data(), acc.p, sizeof(double) * hacc.size(), hipMemcpyDeviceToHost, stream),
-              "copy out");
+    KeptBuf tmp(sizeof(double) * (size_t)N * M * T);
+    results_out(acc.as<double>(), N, M, T, T, nullptr, 3, 3, p->compute_betweenness ? p->betw_scale : 1.0, tmp.as<double>(),
+                out, stream);
     hip_check(hipMemcpyAsync(hreach.data(), reach.p, 4 * T, hipMemcpyDeviceToHost, stream), "copy out");
     hip_check(hipStreamSynchronize(stream), "sync");
-    unpack_acc(hacc, N, M, T, out, nullptr);
-    if (p->compute_betweenness) scale_rows(out, N, T, 3, 3, p->betw_scale);
     if (reach_totals)
       for (uint32_t i = 0; i < T; ++i) reach_totals[i] = hreach[i];
     t_stats.sources = ss.src.size();
@@ -1375,12 +1499,12 @@ static int access_impl(cs_graph *h, uint32_t n_entries, const uint32_t *entry_gr
     std::lock_guard<std::mutex> lk(g.mu);
     DevGraph &dg = device_graph(g, dev);
     DevEdges &de = device_edges(g, dg, speed_m_s);
-    OwnedStream stream;
-    DevBuf d_node_off(4ull * (N + 1)), d_node_mem(4ull * n_assign), d_mem(16ull * n_assign),
+    KeptStream stream;
+    KeptBuf d_node_off(4ull * (N + 1)), d_node_mem(4ull * n_assign), d_mem(16ull * n_assign),
         d_class(4ull * std::max<uint32_t>(n_entries, 1)),
         d_src(4ull * std::max<size_t>(srcs.size(), 1)), d_count(8 * CTN), d_wt(out_div ? 8 : 8 * CTN),
         d_near(8ull * C * N);
-    auto up = [&](DevBuf &d, const void *hsrc, size_t bytes) {
+    auto up = [&](KeptBuf &d, const void *hsrc, size_t bytes) {
       if (bytes) hip_check(hipMemcpyAsync(d.p, hsrc, bytes, hipMemcpyHostToDevice, stream), "copy");
     };
     up(d_node_off, node_off.data(), 4ull * (N + 1));
@@ -1399,7 +1523,7 @@ static int access_impl(cs_graph *h, uint32_t n_entries, const uint32_t *entry_gr
     ao.mem = d_mem.as<uint4>();
     ao.n_shared = n_shared;
     ao.n_groups = n_groups;
-    DevBuf d_stats(8ull * std::max<size_t>((size_t)SM * T * N, 1)),
+    KeptBuf d_stats(8ull * std::max<size_t>((size_t)SM * T * N, 1)),
         d_values(4ull * std::max<size_t>(stats_in ? (size_t)stats_in->n_maps * n_entries : 0, 1));
     if (stats_in) {
       up(d_stats, stat_init.data(), 8ull * SM * T * N);
@@ -1465,36 +1589,29 @@ static int access_impl(cs_graph *h, uint32_t n_entries, const uint32_t *entry_gr
         pending.swap(next);
       }
     }
-    const uint32_t *ip = result_order(g);
+    const uint32_t *d_perm = g.identity_order ? nullptr : dg.perm;
+    KeptBuf tmp(8 * std::max<size_t>({CTN, (size_t)C * N, (size_t)(stats_in ? SM : out_div ? kDivMetrics : 0) * T * N}));
     if (stats_in) {
-      std::vector<double> hs((size_t)SM * T * N);
-      hip_check(hipMemcpyAsync(hs.data(), d_stats.p, 8 * hs.size(), hipMemcpyDeviceToHost, stream), "copy out");
+      results_out(d_stats.as<double>(), N, SM, T, T, d_perm, 0, 0, 1.0, tmp.as<double>(), stats_in->out, stream);
       hip_check(hipStreamSynchronize(stream), "sync");
-      unpack_acc(hs, N, SM, T, stats_in->out, ip);
       t_stats.sources = srcs.size();
       progress_finish(g, N);
       return;
     }
     if (out_div) {
-      DevBuf d_div(8ull * kDivMetrics * T * N);
+      KeptBuf d_div(8ull * kDivMetrics * T * N);
       for (uint32_t t0 = 0; t0 < T; t0 += kMaxT)
         launch_diversity(chunk(t0), C, d_div.as<double>() + (size_t)t0 * N, stream);
-      std::vector<double> hd((size_t)kDivMetrics * T * N);
-      hip_check(hipMemcpyAsync(hd.data(), d_div.p, 8 * hd.size(), hipMemcpyDeviceToHost, stream), "copy out");
+      results_out(d_div.as<double>(), N, kDivMetrics, T, T, d_perm, 0, 0, 1.0, tmp.as<double>(), out_div, stream);
       hip_check(hipStreamSynchronize(stream), "sync");
-      unpack_acc(hd, N, kDivMetrics, T, out_div, ip);
       t_stats.sources = srcs.size();
       progress_finish(g, N);
       return;
     }
-    std::vector<double> hc(CTN), hw(CTN), hn((size_t)C * N);
-    hip_check(hipMemcpyAsync(hc.data(), d_count.p, 8 * CTN, hipMemcpyDeviceToHost, stream), "copy out");
-    hip_check(hipMemcpyAsync(hw.data(), d_wt.p, 8 * CTN, hipMemcpyDeviceToHost, stream), "copy out");
-    hip_check(hipMemcpyAsync(hn.data(), d_near.p, 8ull * C * N, hipMemcpyDeviceToHost, stream), "copy out");
+    results_out(d_count.as<double>(), N, C, T, T, d_perm, 0, 0, 1.0, tmp.as<double>(), out_count, stream);
+    results_out(d_wt.as<double>(), N, C, T, T, d_perm, 0, 0, 1.0, tmp.as<double>(), out_weighted, stream);
+    results_out(d_near.as<double>(), N, C, 1, 1, d_perm, 0, 0, 1.0, tmp.as<double>(), out_nearest, stream);
     hip_check(hipStreamSynchronize(stream), "sync");
-    unpack_acc(hc, N, C, T, out_count, ip);
-    unpack_acc(hw, N, C, T, out_weighted, ip);
-    unpack_acc(hn, N, C, 1, out_nearest, ip);
     t_stats.sources = srcs.size();
     progress_finish(g, N);
   });
@@ -1746,6 +1863,7 @@ int cs_set_tuning(const cs_tuning *t) {
 int cs_release_workspaces(void) {
   return guarded([] {
     release_search_workspaces();
+    kept().release();
     release_angular_workspaces();
   });
 }
@@ -1853,20 +1971,34 @@ int cs_batch_results(cs_batch *b) {
   return guarded([&] {
     if (!b) fail(CS_EINVAL, "batch must not be NULL");
     if (!b->have_results) fail(CS_EINVAL, "the batch has no results: call cs_batch_run first");
-    std::vector<double> hacc(b->acc_words);
     std::vector<uint32_t> hreach(8 * b->jobs.size());
-    if (b->acc_words)
-      hip_check(hipMemcpy(hacc.data(), b->d_acc, 8 * b->acc_words, hipMemcpyDeviceToHost), "copy out");
+    const struct OnDevice {  // the batch's, whichever is current
+      int was = 0;
+      explicit OnDevice(int dev) {
+        hip_check(hipGetDevice(&was), "device");
+        if (was != dev) hip_check(hipSetDevice(dev), "device");
+      }
+      ~OnDevice() { (void)hipSetDevice(was); }
+    } on(b->device);
+    size_t most = 0;
+    for (const cs_batch::JobHost &j : b->jobs) most = std::max(most, (size_t)7 * j.spec.T * j.h->g.n);
+    KeptBuf tmp(8 * most);
     if (!hreach.empty())
       hip_check(hipMemcpy(hreach.data(), b->d_reach, 4 * hreach.size(), hipMemcpyDeviceToHost), "copy out");
     for (size_t i = 0; i < b->jobs.size(); ++i) {
       const cs_batch::JobHost &j = b->jobs[i];
       const uint32_t N = j.h->g.n, T = j.spec.T;
-      unpack_acc_strided(hacc.data() + j.acc_off, N, 7, T, b->NT, j.out, result_order(j.h->g), j.out_T, j.t0);
-      if (j.betw) scale_rows(j.out, N, j.out_T, 5, 6, j.betw_scale, j.t0, T);
+      const uint32_t *d_perm = nullptr;
+      if (!j.h->g.identity_order) {
+        std::lock_guard<std::mutex> lk(j.h->g.mu);
+        d_perm = device_graph(j.h->g, b->device).perm;
+      }
+      results_out(b->d_acc + j.acc_off, N, 7, T, b->NT, d_perm, 5, 6, j.betw ? j.betw_scale : 1.0, tmp.as<double>(), j.out,
+                  b->stream, j.out_T, j.t0);
       if (j.reach)
         for (uint32_t t = 0; t < T; ++t) j.reach[j.t0 + t] = hreach[8 * i + t];
     }
+    hip_check(hipStreamSynchronize(b->stream), "sync");
   });
 }
 

@@ -193,6 +193,8 @@ constexpr uint32_t kProgressSlots = 65536;
 // clears the counts, counts `settled_on_host` sources at once and returns the
 // device address of the counts for the launches to pass on.
 uint32_t *progress_begin(Graph &g, uint64_t settled_on_host);
+// The counts for a launch that keeps n of them (null when it reports none).
+uint32_t *progress_room(uint32_t *progress, uint32_t n);
 // Ends a call's progress at n sources: whatever the kernels have not counted
 // is added on the host (calls that report only on completion count it all).
 void progress_finish(Graph &g, uint64_t n);
@@ -342,6 +344,13 @@ struct ZeroRegion {
   uint64_t *ptr;
   size_t words;
 };
+// Copies accumulators [M][stride][N] out as [M][out_T][N] from threshold t0 on:
+// device node order undone (d_perm; null: none), metrics m0 .. m1 scaled. d_tmp:
+// room for M * T * N where any of it applies. Enqueued; the caller waits.
+void results_out(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32_t stride, const uint32_t *d_perm,
+                 uint32_t m0, uint32_t m1, double scale, double *d_tmp, double *out, hipStream_t stream, uint32_t out_T = 0,
+                 uint32_t t0 = 0);
+
 struct ShortestBatch;
 ShortestBatch *batch_new(std::vector<JobSpec> specs, std::vector<ZeroRegion> zero, uint32_t NT, int device,
                          const Tuning &tune);

@@ -2196,7 +2196,7 @@ void run_jobs(const std::vector<JobSpec> &specs, uint32_t NT, const Tuning &tune
     a.fail_list = d_fail;
     if (tout) a.tout = *tout;
     if (aout) a.acc = *aout;
-    a.progress = waves <= kProgressSlots ? progress : nullptr;
+    a.progress = progress_room(progress, waves);
     hip_check(hipEventRecord(e0, stream), "event record");
     launch_nt<MODE>(NT, waves / wpb, block, lds, stream, a);
     hip_check(hipGetLastError(), "k_search launch");
@@ -2544,6 +2544,43 @@ __global__ void k_map_ids(uint32_t *out, const uint32_t *in, const uint32_t *per
 __global__ void k_gather_u8(uint8_t *out, const uint8_t *in, const uint32_t *orig, uint32_t N) {
   const uint32_t d = blockIdx.x * blockDim.x + threadIdx.x;
   if (d < N) out[d] = in[orig[d]];
+}
+
+// Results as the caller gets them: dst[m][t][v] = src[m][t of stride][perm[v]],
+// metrics m0 .. m1 scaled. Reads are scattered within a row (the order is a
+// space-filling curve of the nodes), writes are whole lines. The copy out is all
+// that is left: 7 MB (32,400 nodes, 28 rows) cost a call 2.3 ms less than the
+// same reordering on the host.
+__global__ void k_results(double *dst, const double *src, const uint32_t *perm, uint32_t N, uint32_t T, uint32_t stride,
+                          uint32_t m0, uint32_t m1, double scale, uint32_t row0) {
+  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x, row = row0 + blockIdx.y, m = row / T, t = row % T;
+  if (v >= N) return;
+  double x = src[((size_t)m * stride + t) * N + (perm ? perm[v] : v)];
+  if (scale != 1.0 && m >= m0 && m <= m1) x *= scale;
+  dst[(size_t)row * N + v] = x;
+}
+
+void results_out(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32_t stride, const uint32_t *d_perm,
+                 uint32_t m0, uint32_t m1, double scale, double *d_tmp, double *out, hipStream_t stream, uint32_t out_T,
+                 uint32_t t0) {
+  if (!N || !M || !T) return;
+  if (out_T == 0) out_T = T;
+  const double *from = d_acc;
+  if (d_perm || stride != T || scale != 1.0) {
+    for (uint32_t row = 0; row < M * T; row += 32768)
+      hipLaunchKernelGGL(k_results, dim3((N + 255) / 256, std::min(M * T - row, 32768u)), dim3(256), 0, stream, d_tmp, d_acc,
+                         d_perm, N, T, stride, m0, m1, scale, row);
+    hip_check(hipGetLastError(), "k_results launch");
+    from = d_tmp;
+  }
+  const size_t rows = (size_t)T * N;
+  if (out_T == T) {
+    hip_check(hipMemcpyAsync(out, from, 8 * rows * M, hipMemcpyDeviceToHost, stream), "copy out");
+    return;
+  }
+  for (uint32_t m = 0; m < M; ++m)
+    hip_check(hipMemcpyAsync(out + ((size_t)m * out_T + t0) * N, from + m * rows, 8 * rows, hipMemcpyDeviceToHost, stream),
+              "copy out");
 }
 
 // dst[r][orig[d]] += src[r][d] over rows x N: orig is a permutation, so every
@@ -2965,7 +3002,7 @@ void launch_access_lists(const AccessOut &out, const uint32_t *d_src, const uint
     a.next = d_ctl.p;
     a.n_fail = d_ctl.p + 1;
     a.fail_list = d_fail.p;
-    a.progress = waves <= kProgressSlots ? progress : nullptr;
+    a.progress = progress_room(progress, waves);
     hipEvent_t e0, e1;
     hip_check(hipEventCreate(&e0), "event");
     hip_check(hipEventCreate(&e1), "event");
