@@ -985,7 +985,10 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
     const int dev = current_device();
     const CallSpec spec = make_spec(p, 0, chunk_len(p->n_thresholds, 0));
     SourceSet ss = source_set(g, p);
-    to_device_sources(g, ss);
+    // many sources are put in device order on the device
+    g.order_frozen = true;
+    const bool reorder = !g.identity_order && ss.src.size() >= kOrderOnDevice;
+    if (!reorder) to_device_sources(g, ss);
     const std::vector<uint8_t> elig = to_device_u8(g, p->eligible);
     const uint32_t N = g.n, T = p->n_thresholds, M = 7;
     KeptStream stream;
@@ -993,10 +996,15 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
         d_wt(4 * ss.src.size()), d_cyc(4 * ss.src.size()), d_elig(N);
     hip_check(hipMemsetAsync(acc.p, 0, sizeof(double) * (size_t)N * M * T, stream), "memset");
     hip_check(hipMemsetAsync(reach.p, 0, 4 * T, stream), "memset");
+    const size_t n_raw = reorder ? ss.src.size() : 0;
+    KeptBuf r_src(4 * n_raw), r_wt(4 * n_raw), r_cyc(4 * n_raw), r_tmp(reorder ? 4 * order_scratch(N) : 0);
     if (!ss.src.empty()) {
-      hip_check(hipMemcpyAsync(d_src.p, ss.src.data(), 4 * ss.src.size(), hipMemcpyHostToDevice, stream), "copy");
-      hip_check(hipMemcpyAsync(d_wt.p, ss.wt.data(), 4 * ss.wt.size(), hipMemcpyHostToDevice, stream), "copy");
-      hip_check(hipMemcpyAsync(d_cyc.p, ss.cyc.data(), 4 * ss.cyc.size(), hipMemcpyHostToDevice, stream), "copy");
+      hip_check(hipMemcpyAsync(reorder ? r_src.p : d_src.p, ss.src.data(), 4 * ss.src.size(), hipMemcpyHostToDevice, stream),
+                "copy");
+      hip_check(hipMemcpyAsync(reorder ? r_wt.p : d_wt.p, ss.wt.data(), 4 * ss.wt.size(), hipMemcpyHostToDevice, stream),
+                "copy");
+      hip_check(hipMemcpyAsync(reorder ? r_cyc.p : d_cyc.p, ss.cyc.data(), 4 * ss.cyc.size(), hipMemcpyHostToDevice, stream),
+                "copy");
     }
     hip_check(hipMemcpyAsync(d_elig.p, elig.data(), N, hipMemcpyHostToDevice, stream), "copy");
     const uint32_t *d_perm = nullptr;
@@ -1006,6 +1014,9 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
       DevEdges &de = device_edges(g, dg, spec.speed);
       if (!g.identity_order) d_perm = dg.perm;
       run_shortest_checks(g, p);
+      if (reorder)
+        order_sources(r_src.as<uint32_t>(), r_wt.as<float>(), r_cyc.as<float>(), (uint32_t)n_raw, dg.perm, N,
+                      r_tmp.as<uint32_t>(), d_src.as<uint32_t>(), d_wt.as<float>(), d_cyc.as<float>(), stream);
       uint32_t *prog = progress_begin(g, p->n_sources - ss.src.size());
       // a call of several threshold chunks reports progress in its last one
       for (uint32_t t0 = 0; t0 < T; t0 += kMaxT)
@@ -1193,16 +1204,25 @@ int cs_segment_centrality(cs_graph *h, const cs_params *p, double *out) {
     std::vector<uint32_t> srcs;
     for (uint32_t i = 0; i < p->n_sources; ++i)
       if (g.live[p->sources[i]]) srcs.push_back(p->sources[i]);
-    to_device_ids(g, srcs);
-    std::sort(srcs.begin(), srcs.end());
+    g.order_frozen = true;
+    const bool reorder = !g.identity_order && srcs.size() >= kOrderOnDevice;
+    if (!reorder) {
+      to_device_ids(g, srcs);
+      std::sort(srcs.begin(), srcs.end());
+    }
     std::lock_guard<std::mutex> lk(g.mu);
     DevGraph &dg = device_graph(g, dev);
     DevEdges &de = device_edges(g, dg, p->speed_m_s);
     KeptStream stream;
-    KeptBuf acc(sizeof(double) * (size_t)N * M * T), d_src(4 * srcs.size());
+    KeptBuf acc(sizeof(double) * (size_t)N * M * T), d_src(4 * srcs.size()), r_src(reorder ? 4 * srcs.size() : 0),
+        r_tmp(reorder ? 4 * order_scratch(N) : 0);
     hip_check(hipMemsetAsync(acc.p, 0, sizeof(double) * (size_t)N * M * T, stream), "memset");
     if (!srcs.empty())
-      hip_check(hipMemcpyAsync(d_src.p, srcs.data(), 4 * srcs.size(), hipMemcpyHostToDevice, stream), "copy");
+      hip_check(hipMemcpyAsync(reorder ? r_src.p : d_src.p, srcs.data(), 4 * srcs.size(), hipMemcpyHostToDevice, stream),
+                "copy");
+    if (reorder)
+      order_sources(r_src.as<uint32_t>(), nullptr, nullptr, (uint32_t)srcs.size(), dg.perm, N, r_tmp.as<uint32_t>(),
+                    d_src.as<uint32_t>(), nullptr, nullptr, stream);
     uint32_t *prog = progress_begin(g, p->n_sources - srcs.size());
     for (uint32_t t0 = 0; t0 < T; t0 += kMaxT)
       launch_segment(g, dg, de, make_spec(p, t0, chunk_len(T, t0)), d_src.as<uint32_t>(), (uint32_t)srcs.size(),
@@ -1470,8 +1490,12 @@ static int access_impl(cs_graph *h, uint32_t n_entries, const uint32_t *entry_gr
     std::vector<uint32_t> srcs;
     for (uint32_t v = 0; v < N; ++v)
       if (g.live[v]) srcs.push_back(v);
-    to_device_ids(g, srcs);
-    std::sort(srcs.begin(), srcs.end());
+    g.order_frozen = true;
+    const bool reorder = !g.identity_order && srcs.size() >= kOrderOnDevice;
+    if (!reorder) {
+      to_device_ids(g, srcs);
+      std::sort(srcs.begin(), srcs.end());
+    }
     AccessOut ao;
     ao.N = N;
     ao.tstride = T;
@@ -1511,7 +1535,11 @@ static int access_impl(cs_graph *h, uint32_t n_entries, const uint32_t *entry_gr
     up(d_node_mem, node_mem.data(), 4ull * n_assign);
     up(d_mem, mem.data(), 16ull * n_assign);
     if (entry_class) up(d_class, entry_class, 4ull * n_entries);
-    up(d_src, srcs.data(), 4ull * srcs.size());
+    KeptBuf r_src(reorder ? 4 * srcs.size() : 0), r_tmp(reorder ? 4 * order_scratch(N) : 0);
+    up(reorder ? r_src : d_src, srcs.data(), 4ull * srcs.size());
+    if (reorder)
+      order_sources(r_src.as<uint32_t>(), nullptr, nullptr, (uint32_t)srcs.size(), dg.perm, N, r_tmp.as<uint32_t>(),
+                    d_src.as<uint32_t>(), nullptr, nullptr, stream);
     {
       const std::vector<double> nan_rows((size_t)C * N, std::nan(""));  // NaN bits: no entry yet
       up(d_near, nan_rows.data(), 8ull * C * N);

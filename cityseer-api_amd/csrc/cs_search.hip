@@ -2546,6 +2546,96 @@ __global__ void k_gather_u8(uint8_t *out, const uint8_t *in, const uint32_t *ori
   if (d < N) out[d] = in[orig[d]];
 }
 
+// A call's sources in device node order, the order a launch's waves share rows
+// in: counted per device node, the counts scanned, each source placed. Five
+// launches of a few us; sorting 30,406 sources on the host took 1.4 ms of a 5.6
+// ms call. (Sources named twice stand side by side in either order.)
+constexpr uint32_t kOrderSpan = 2048;  // counts a workgroup of 256 scans
+__device__ __forceinline__ uint32_t scan_block(uint32_t x, uint32_t *wsum) {  // exclusive, 256 threads
+  const uint32_t lane = lane_id(), w = threadIdx.x / kWave;
+  const uint32_t incl = __ockl_wfscan_add_u32(x, true);
+  if (lane == kWave - 1) wsum[w] = incl;
+  __syncthreads();
+  uint32_t before = incl - x;
+  for (uint32_t k = 0; k < w; ++k) before += wsum[k];
+  __syncthreads();
+  return before;
+}
+
+__global__ void k_order_count(const uint32_t *src, uint32_t n, const uint32_t *perm, uint32_t *count) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) atomicAdd(&count[perm[src[i]]], 1u);
+}
+
+__global__ __launch_bounds__(256) void k_order_sums(const uint32_t *count, uint32_t N, uint32_t *sums) {
+  __shared__ uint32_t wsum[4];
+  uint32_t x = 0;
+  for (uint32_t k = 0; k < kOrderSpan; k += 256) {
+    const uint32_t d = blockIdx.x * kOrderSpan + k + threadIdx.x;
+    if (d < N) x += count[d];
+  }
+  const uint32_t before = scan_block(x, wsum);
+  if (threadIdx.x == 255) sums[blockIdx.x] = before + x;
+}
+
+__global__ __launch_bounds__(256) void k_order_scan(uint32_t *sums, uint32_t nb) {
+  __shared__ uint32_t wsum[4], total;
+  uint32_t base = 0;
+  for (uint32_t k = 0; k < nb; k += 256) {
+    const uint32_t i = k + threadIdx.x, x = i < nb ? sums[i] : 0u;
+    const uint32_t before = scan_block(x, wsum);
+    if (i < nb) sums[i] = base + before;
+    if (threadIdx.x == 255) total = before + x;
+    __syncthreads();
+    base += total;
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(256) void k_order_offsets(uint32_t *count, uint32_t N, const uint32_t *sums) {
+  __shared__ uint32_t wsum[4];
+  constexpr uint32_t kEach = kOrderSpan / 256;
+  const uint32_t d0 = blockIdx.x * kOrderSpan + threadIdx.x * kEach;
+  uint32_t c[kEach], x = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kEach; ++k) {
+    c[k] = d0 + k < N ? count[d0 + k] : 0u;
+    x += c[k];
+  }
+  uint32_t at = sums[blockIdx.x] + scan_block(x, wsum);
+#pragma unroll
+  for (uint32_t k = 0; k < kEach; ++k) {
+    if (d0 + k < N) count[d0 + k] = at;
+    at += c[k];
+  }
+}
+
+__global__ void k_order_place(const uint32_t *src, const float *wt, const float *cyc, uint32_t n, const uint32_t *perm,
+                              uint32_t *offset, uint32_t *o_src, float *o_wt, float *o_cyc) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t d = perm[src[i]], at = atomicAdd(&offset[d], 1u);
+  o_src[at] = d;
+  if (wt) o_wt[at] = wt[i];
+  if (cyc) o_cyc[at] = cyc[i];
+}
+
+size_t order_scratch(uint32_t N) { return N + (N + kOrderSpan - 1) / kOrderSpan; }
+
+void order_sources(const uint32_t *src, const float *wt, const float *cyc, uint32_t n, const uint32_t *d_perm, uint32_t N,
+                   uint32_t *tmp, uint32_t *o_src, float *o_wt, float *o_cyc, hipStream_t stream) {
+  const uint32_t nb = (N + kOrderSpan - 1) / kOrderSpan;
+  uint32_t *sums = tmp + N;
+  const dim3 block(256), per_src((n + 255) / 256);
+  hip_check(hipMemsetAsync(tmp, 0, 4ull * N, stream), "memset");
+  hipLaunchKernelGGL(k_order_count, per_src, block, 0, stream, src, n, d_perm, tmp);
+  hipLaunchKernelGGL(k_order_sums, dim3(nb), block, 0, stream, tmp, N, sums);
+  hipLaunchKernelGGL(k_order_scan, dim3(1), block, 0, stream, sums, nb);
+  hipLaunchKernelGGL(k_order_offsets, dim3(nb), block, 0, stream, tmp, N, sums);
+  hipLaunchKernelGGL(k_order_place, per_src, block, 0, stream, src, wt, cyc, n, d_perm, tmp, o_src, o_wt, o_cyc);
+  hip_check(hipGetLastError(), "source order launch");
+}
+
 // Results as the caller gets them: dst[m][t][v] = src[m][t of stride][perm[v]],
 // metrics m0 .. m1 scaled. Reads are scattered within a row (the order is a
 // space-filling curve of the nodes), writes are whole lines. The copy out is all
