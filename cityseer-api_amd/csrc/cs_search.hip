@@ -2639,7 +2639,7 @@ void order_sources(const uint32_t *src, const float *wt, const float *cyc, uint3
 // Results as the caller gets them: dst[m][t][v] = src[m][t of stride][perm[v]],
 // metrics m0 .. m1 scaled. Reads are scattered within a row (the order is a
 // space-filling curve of the nodes), writes are whole lines. The copy out is all
-// that is left: 7 MB (32,400 nodes, 28 rows) cost a call 2.3 ms less than the
+// that is left: 9 MB (40,000 nodes, 28 rows) cost a call 2.3 ms less than the
 // same reordering on the host.
 __global__ void k_results(double *dst, const double *src, const uint32_t *perm, uint32_t N, uint32_t T, uint32_t stride,
                           uint32_t m0, uint32_t m1, double scale, uint32_t row0) {
