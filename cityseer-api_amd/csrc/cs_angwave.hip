@@ -194,9 +194,11 @@ __device__ __forceinline__ uint32_t page_of(const WaveArgs &a, const Search &q, 
 }
 
 // The page of node v, met for the first time: all its states unreached. False
-// without room.
+// without room, and then nothing is touched: a superpage is only ever taken with
+// a page of it, which is how the clean-up after a search finds its table byte.
 __device__ __forceinline__ bool open_page(const WaveArgs &a, Search &q, uint32_t v) {
   const uint32_t lane = lane_id(), rs = a.ss - kPage;
+  if (q.np == a.P) return false;
   uint32_t sp = uniform(q.pt[v >> a.ss]);
   if (sp == kNoSuper) {
     if (q.nq == a.Q) return false;
@@ -205,7 +207,6 @@ __device__ __forceinline__ bool open_page(const WaveArgs &a, Search &q, uint32_t
     if (lane == 0) q.pt[v >> a.ss] = (uint8_t)sp;
     order();
   }
-  if (q.np == a.P) return false;
   const uint32_t id = q.np++;
   if (lane < (1u << kPage)) {
     *reinterpret_cast<float2 *>(&q.R[2 * ((id << kPage) + lane)]) = make_float2(INFINITY, INFINITY);

@@ -2,7 +2,8 @@
 everywhere (one at a time, and many at one route), streets cut into short straight pieces (no two
 states safe together), crossings of more than four streets (longer rows than one state's lanes),
 more thresholds than one back-propagation pass holds, and searches that outgrow the room the
-probed sources asked for (a dense knot in a sparse network)."""
+probed sources asked for (a dense knot in a sparse network; many dense cores, where searches run out
+of pages at a run of nodes met for the first time and their waves go on to other sources)."""
 
 from __future__ import annotations
 
@@ -69,3 +70,34 @@ def test_matches_oracle(name, distances):
     assert_close(got, ref, name)
     if name == "knot":
         assert _native.last_stats()["retries"] > 0
+
+
+def _cores(side, across, size):
+    """A lattice at 100 m with across x across lattices at 4 m hung on it."""
+    a = mock.perturbed_lattice(side, seed=5)
+    x, y, edges, length, k = [a.x], [a.y], [a.edges], [a.length], len(a.x)
+    for i in range(across):
+        for j in range(across):
+            b = mock.perturbed_lattice(size, spacing=4.0, jitter=1.0, seed=6 + across * i + j)
+            c = int(np.argmin(np.hypot(a.x - 100.0 * side * (i + 0.5) / across, a.y - 100.0 * side * (j + 0.5) / across)))
+            x.append(b.x + a.x[c] + 20.0)
+            y.append(b.y + a.y[c] + 20.0)
+            edges += [b.edges + k, np.array([[c, k]])]
+            length += [b.length, np.float32([30.0])]
+            k += len(b.x)
+    return mock.Lattice(x=np.concatenate(x), y=np.concatenate(y), edges=np.concatenate(edges),
+                        length=np.concatenate(length).astype(np.float32))
+
+
+def test_waves_search_on_after_running_out_of_pages():
+    """12,518 dual nodes, three sources a wave: by the layout's arithmetic (the probed sources reach 448
+    nodes: 74 pages, 16 runs of 64 nodes) two thirds run out of pages, some 360 of them at a run of
+    nodes met for the first time."""
+    O.set_heap_mode(False)
+    ns = mock.network_structure_from_lattice(mock.lattice_dual(_cores(70, 4, 12)))
+    say(f"angular search, dense cores: {ns.node_count()} dual nodes")
+    got = stack(ns.centrality_simplest(distances=[1200]), SIMPLEST, [1200])
+    assert _native.last_stats()["retries"] > 1000
+    ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest([1200], n_threads=8)
+    assert np.array_equal(got[0], ref[0])
+    assert_close(got, ref, "dense cores")
