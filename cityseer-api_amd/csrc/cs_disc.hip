@@ -1033,7 +1033,9 @@ __global__ void k_disc_zero(uint64_t *p, uint32_t n) {
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // The graph's rows for this kernel, built once per speed, on the device from the
-// edge arrays it holds.
+// edge arrays it holds. They are there when this returns: another call may read
+// them on its own stream as soon as the caller lets go of disc_mu (a batch that
+// plans holds no other lock of the graph), and `tmp` may go to another call.
 DiscGraph &disc_graph(const Graph &g, const DevGraph &dg, DevEdges &de, DevVec &tmp, hipStream_t stream) {
   if (de.disc) return *de.disc;
   auto w = std::make_unique<DiscGraph>();
@@ -1057,6 +1059,7 @@ DiscGraph &disc_graph(const Graph &g, const DevGraph &dg, DevEdges &de, DevVec &
       hip_check(hipMalloc(&w->row, sizeof(uint4) * n * w->blocks * kQuad), "hipMalloc rows");
       hipLaunchKernelGGL(k_disc_rows, grid, block, 0, stream, dg.rows, de.rev_adj, de.fwd_adj, n, w->blocks, meas, w->row);
       hip_check(hipGetLastError(), "rows launch");
+      hip_check(hipStreamSynchronize(stream), "sync");
     }
   }
   de.disc = std::move(w);
