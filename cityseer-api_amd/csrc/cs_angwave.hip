@@ -1002,11 +1002,9 @@ WaveWorkspace &wave_ws(int device) {
 }
 
 template <typename T>
-T *to_device(const std::vector<T> &v) {
-  T *p = nullptr;
-  hip_check(hipMalloc(&p, sizeof(T) * std::max<size_t>(v.size(), 1)), "hipMalloc angular rows");
-  if (!v.empty()) hip_check(hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice), "upload");
-  return p;
+void to_device(const std::vector<T> &v, T **p) {
+  hip_check(hipMalloc(p, sizeof(T) * std::max<size_t>(v.size(), 1)), "hipMalloc angular rows");
+  if (!v.empty()) hip_check(hipMemcpy(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice), "upload");
 }
 
 uint32_t bits(float x) {
@@ -1069,13 +1067,13 @@ AngWaveGraph &wave_graph(Graph &g, DevEdges &de) {
           }
         }
       }
-    w->row = to_device(row);
-    w->row_wm = to_device(row_wm);
-    w->spill = to_device(spill);
-    w->spill_wm = to_device(spill_wm);
-    w->wm = to_device(wm);
-    w->perm = to_device(perm);
-    w->orig = to_device(orig);
+    to_device(row, &w->row);
+    to_device(row_wm, &w->row_wm);
+    to_device(spill, &w->spill);
+    to_device(spill_wm, &w->spill_wm);
+    to_device(wm, &w->wm);
+    to_device(perm, &w->perm);
+    to_device(orig, &w->orig);
   }
   w->usable = ok;
   de.ang_wave = std::move(w);
@@ -1181,9 +1179,8 @@ bool wave_layout(WaveArgs &a, uint32_t N, uint32_t nodes, const uint32_t *pages,
 
 }  // namespace
 
-void free_angular_wave(AngWaveGraph &w) {
-  for (void *p : {(void *)w.row, (void *)w.row_wm, (void *)w.spill, (void *)w.spill_wm, (void *)w.wm, (void *)w.perm,
-                  (void *)w.orig})
+AngWaveGraph::~AngWaveGraph() {
+  for (void *p : {(void *)row, (void *)row_wm, (void *)spill, (void *)spill_wm, (void *)wm, (void *)perm, (void *)orig})
     (void)hipFree(p);
 }
 

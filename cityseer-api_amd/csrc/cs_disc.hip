@@ -1602,7 +1602,7 @@ uint32_t disc_nodes(const DevEdges &de, float maxsec) {
   return n > kProbeStop ? 4 * 16384u : n + n / 4;
 }
 
-void free_disc(DiscGraph &w) { (void)hipFree(w.row); }
+DiscGraph::~DiscGraph() { (void)hipFree(row); }
 
 void release_disc_workspaces() {
   std::lock_guard<std::mutex> lk(g_disc_mu);

@@ -170,8 +170,8 @@ void free_edges(DevEdges &d) {
   (void)hipFree(d.fwd_eid);
   (void)hipFree(d.ang_adj);
   (void)hipFree(d.ang_srow);
-  if (d.ang_wave) free_angular_wave(*d.ang_wave);
-  if (d.disc) free_disc(*d.disc);
+  d.ang_wave.reset();
+  d.disc.reset();
 }
 
 }  // namespace

@@ -88,6 +88,8 @@ struct AngWaveGraph {
     bool chains = false;  // most nodes lead on to others (streets cut into short pieces)
   };
   std::map<float, Reach> reach;
+  AngWaveGraph() = default;
+  ~AngWaveGraph();  // (also of one whose building failed half way)
 };
 
 // What the LDS shortest search (cs_disc.hip) reads of a graph.
@@ -104,6 +106,8 @@ struct DiscGraph {
     uint32_t pages[10] = {0};
   };
   std::map<float, Reach> reach;
+  DiscGraph() = default;
+  ~DiscGraph();
 };
 
 // Speed-dependent device edge arrays for one (device, speed).
@@ -328,7 +332,6 @@ void disc_batch_collect(const DiscBatch &b, hipStream_t stream, cs_stats &st, st
 // Nodes of a search up to maxsec as far as probed searches tell, with a quarter
 // more (0: none were).
 uint32_t disc_nodes(const DevEdges &de, float maxsec);
-void free_disc(DiscGraph &w);
 void release_disc_workspaces();
 
 // All sources of all jobs in one persistent launch, or only `items`
@@ -453,7 +456,6 @@ void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<u
 std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items,
                                         uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress,
                                         bool *done);
-void free_angular_wave(AngWaveGraph &w);
 void release_angular_wave_workspaces();
 
 void launch_simplest(Graph &g, DevGraph &dg, DevEdges &de, const CallSpec &cs,
