@@ -7,6 +7,8 @@ of pages at a run of nodes met for the first time and their waves go on to other
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -101,3 +103,25 @@ def test_waves_search_on_after_running_out_of_pages():
     ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest([1200], n_threads=8)
     assert np.array_equal(got[0], ref[0])
     assert_close(got, ref, "dense cores")
+
+
+def test_lane_workspace_does_not_creep():
+    """A network whose lanes are as many as a share of the memory holds: repeated calls run the same number
+    of waves, in the same workspace."""
+    ns = mock.network_structure_from_lattice(mock.lattice_dual(mock.perturbed_lattice(240, seed=74)))
+    lib, tuning = _native.load(), _native.CsTuning()
+    _native.check(lib.cs_get_tuning(ctypes.byref(tuning)))
+    lanes, tuning.simplest_lanes = tuning.simplest_lanes, 64
+    _native.check(lib.cs_set_tuning(ctypes.byref(tuning)))
+    try:
+        waves = []
+        for k in range(3):
+            say(f"{ns.node_count()} dual nodes, one lane per source, call {k}")
+            ns.centrality_simplest(distances=[150])
+            waves.append(_native.last_stats()["waves"])
+    finally:
+        tuning.simplest_lanes = lanes
+        _native.check(lib.cs_set_tuning(ctypes.byref(tuning)))
+        _native.check(lib.cs_release_workspaces())
+    assert waves[0] * 64 < ns.node_count()
+    assert waves[1:] == waves[:-1]
