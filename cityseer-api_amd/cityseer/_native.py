@@ -214,6 +214,7 @@ _SIGNATURES = {
         [ctypes.c_void_p, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_float, ctypes.c_float, _f32p, _f32p, _f64p,
          _u32p, _u32p, ctypes.c_uint32],
     ),
+    "cs_last_lds_searches": (ctypes.c_uint64, []),
     "cs_last_stats": (ctypes.c_int, [ctypes.POINTER(CsStats)]),
     "cs_set_tuning": (ctypes.c_int, [ctypes.POINTER(CsTuning)]),
     "cs_get_tuning": (ctypes.c_int, [ctypes.POINTER(CsTuning)]),
@@ -291,3 +292,8 @@ def last_stats() -> dict:
     st = CsStats()
     check(load().cs_last_stats(ctypes.byref(st)))
     return {name: getattr(st, name) for name, _ in CsStats._fields_}
+
+
+def last_lds_searches() -> int:
+    """Searches of this thread's last call that ran to their end in LDS."""
+    return int(load().cs_last_lds_searches())

@@ -1347,6 +1347,7 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
     st.kernel_ms += ms;
     st.waves = std::max<uint32_t>(st.waves, waves);
     const uint32_t n_failed = hctl[kXcd];
+    thread_lds_searches() += n_list - n_failed;
     std::vector<uint2> left(n_failed);
     if (n_failed) {
       std::vector<uint32_t> fl(n_failed);

@@ -1465,6 +1465,7 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
     st.edges_scanned += stv[1];
     st.within_sum += stv[2];
     const uint32_t n_failed = h[kXcd];
+    thread_lds_searches() += d.n - n_failed;
     if (!n_failed) continue;
     if (h[kXcd + 1] & kFailInternal) fail(CS_EINTERNAL, "search invariant violated (settle order)");
     std::vector<uint32_t> fl(n_failed);
@@ -1582,6 +1583,7 @@ void disc_batch_collect(const DiscBatch &b, hipStream_t stream, cs_stats &st, st
     st.edges_scanned += stv[1];
     st.within_sum += stv[2];
     const uint32_t n_failed = c[kXcd];
+    thread_lds_searches() += p.d.n - n_failed;
     if (!n_failed) continue;
     if (c[kXcd + 1] & kFailInternal) fail(CS_EINTERNAL, "search invariant violated (settle order)");
     std::vector<uint32_t> fl(n_failed);

@@ -17,6 +17,11 @@ namespace cs {
 namespace {
 thread_local std::string t_err;
 thread_local cs_stats t_stats;
+thread_local uint64_t t_lds_searches;
+void reset_stats() {
+  t_stats = cs_stats{};
+  t_lds_searches = 0;
+}
 }  // namespace
 
 void fail(int code, const std::string &msg) { throw Error{code, msg}; }
@@ -30,6 +35,7 @@ void hip_check(hipError_t e, const char *what) {
 }
 
 cs_stats &thread_stats() { return t_stats; }
+uint64_t &thread_lds_searches() { return t_lds_searches; }
 
 // Tobler slope penalty and edge travel seconds (centrality.rs:970-1007).
 float edge_seconds(const Graph &g, uint32_t from, uint32_t to, uint32_t e, float speed,
@@ -990,9 +996,11 @@ int cs_last_stats(cs_stats *out) {
   return CS_OK;
 }
 
+uint64_t cs_last_lds_searches(void) { return t_lds_searches; }
+
 int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_t *reach_totals) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!h || !out) fail(CS_EINVAL, "graph and out must not be NULL");
     Graph &g = h->g;
@@ -1058,7 +1066,7 @@ int cs_centrality_shortest(cs_graph *h, const cs_params *p, double *out, uint32_
 int cs_centrality_shortest_device(cs_graph *h, const cs_params *p, const float *d_cycles_wt, double *d_acc,
                                   uint32_t *d_reach, void *stream_ptr) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!h || !p || !d_acc) fail(CS_EINVAL, "graph, params and d_acc must not be NULL");
     Graph &g = h->g;
@@ -1090,7 +1098,7 @@ int cs_centrality_shortest_device(cs_graph *h, const cs_params *p, const float *
 int cs_betweenness_od_shortest(cs_graph *h, const cs_params *p, uint32_t n_pairs, const uint32_t *origins,
                                const uint32_t *destinations, const float *weights, double *out) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!h || !p || !out) fail(CS_EINVAL, "graph, params and out must not be NULL");
     if (n_pairs && (!origins || !destinations || !weights))
@@ -1203,7 +1211,7 @@ int cs_betweenness_od_shortest(cs_graph *h, const cs_params *p, uint32_t n_pairs
 
 int cs_segment_centrality(cs_graph *h, const cs_params *p, double *out) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!h || !out) fail(CS_EINVAL, "graph and out must not be NULL");
     Graph &g = h->g;
@@ -1253,7 +1261,7 @@ int cs_segment_centrality(cs_graph *h, const cs_params *p, double *out) {
 
 int cs_centrality_simplest(cs_graph *h, const cs_params *p, double *out, uint32_t *reach_totals) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!h || !out) fail(CS_EINVAL, "graph and out must not be NULL");
     Graph &g = h->g;
@@ -1414,7 +1422,7 @@ static int access_impl(cs_graph *h, uint32_t n_entries, const uint32_t *entry_gr
                        double *out_weighted, double *out_nearest, double *out_div,
                        const StatsIn *stats_in = nullptr) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!h) fail(CS_EINVAL, "graph must not be NULL");
     Graph &g = h->g;
@@ -1980,7 +1988,7 @@ int cs_batch_set_tuning(cs_batch *b, const cs_tuning *t) {
 
 int cs_batch_autotune(cs_batch *b, double sample_fraction, cs_tuning *chosen) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!b) fail(CS_EINVAL, "batch must not be NULL");
     if (!(sample_fraction > 0.0 && sample_fraction <= 1.0)) fail(CS_EINVAL, "sample_fraction must be in (0, 1]");
@@ -1995,7 +2003,7 @@ int cs_batch_autotune(cs_batch *b, double sample_fraction, cs_tuning *chosen) {
 
 int cs_batch_run(cs_batch *b) {
   const auto t0 = std::chrono::steady_clock::now();
-  t_stats = cs_stats{};
+  reset_stats();
   int rc = guarded([&] {
     if (!b) fail(CS_EINVAL, "batch must not be NULL");
     b->build();

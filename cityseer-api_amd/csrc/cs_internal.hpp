@@ -224,6 +224,7 @@ DevEdges *find_device_edges(DevGraph &dg, float speed);
 
 // Per-call statistics (thread-local).
 cs_stats &thread_stats();
+uint64_t &thread_lds_searches();  // of the same call: searches that ran to their end in LDS
 
 // ----------------------------------------------------------------------
 // Kernel launchers (cs_search.hip)

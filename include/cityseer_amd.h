@@ -370,6 +370,10 @@ typedef struct cs_stats {
 /* Statistics of the calling thread's last compute call. */
 int cs_last_stats(cs_stats *out);
 
+/* Searches of the same call that ran to their end with their state in LDS (a
+ * source counts once per eight thresholds); the others ran in scratch memory. */
+uint64_t cs_last_lds_searches(void);
+
 /* ---------------------------------------------------------------------- */
 /* Launch shape and batching                                              */
 /* ---------------------------------------------------------------------- */

@@ -67,11 +67,13 @@ def test_matches_oracle(name, distances):
     ns = mock.network_structure_from_lattice(mock.lattice_dual(primal))
     say(f"angular search, {name}: {ns.node_count()} dual nodes, {distances} m")
     got = stack(ns.centrality_simplest(distances=distances), SIMPLEST, distances)
+    stats = _native.last_stats()
+    assert _native.last_lds_searches() == stats["sources"]
     ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest(distances)
     assert np.array_equal(got[0], ref[0])
     assert_close(got, ref, name)
     if name == "knot":
-        assert _native.last_stats()["retries"] > 0
+        assert stats["retries"] > 0
 
 
 def _cores(side, across, size):

@@ -77,7 +77,7 @@ def test_matches_oracle(name, distances, kw):
         ns = mock.network_structure_from_lattice(make[name]())
     say(f"shortest search, {name}: {ns.node_count()} nodes, {distances} m {kw}")
     res = ns.centrality_shortest(distances=distances, **kw)
-    stats = _native.last_stats()
+    stats, in_lds = _native.last_stats(), _native.last_lds_searches()
     plan = ns._sampling_plan(None, None, None, kw.get("source_indices"))
     ref, _ = OracleGraph.from_network_structure(ns).centrality_shortest(
         distances, closeness=kw.get("compute_closeness", True), betweenness=kw.get("compute_betweenness", True),
@@ -85,6 +85,8 @@ def test_matches_oracle(name, distances, kw):
     got = stack(res, SHORTEST_KEYS, distances)
     assert np.array_equal(got[0], ref[0])
     assert_close(got, ref, name)
+    # which search ran: rows of more than 16 neighbours have no place in LDS
+    assert in_lds == (0 if name == "star18" else stats["sources"])
     if name == "knot":
         assert stats["retries"] > 0
 
@@ -98,6 +100,7 @@ def test_large_reach_is_searched_once():
     say(f"shortest search, large reach: {n} nodes, {len(src)} sources")
     res = ns.centrality_shortest(distances=[600, 9000], source_indices=src)
     stats = _native.last_stats()
+    assert _native.last_lds_searches() == 0
     assert stats["nodes_reached"] > 16384 * len(src) and stats["retries"] == 0
     plan = ns._sampling_plan(None, None, None, src)
     ref, _ = OracleGraph.from_network_structure(ns).centrality_shortest(
@@ -120,6 +123,8 @@ def test_batch_mixes_searches_and_replays():
             say(f"batch of {len(nets)} networks, run {k}")
             stats = batch.run()
             assert stats["retries"] > 0
+            in_lds = _native.last_lds_searches()
+            assert 0 < in_lds < stats["sources"] - nets[1].node_count()
             for i, (res, d) in enumerate(zip(batch.results(), asked)):
                 got = stack(res, SHORTEST_KEYS, d)
                 assert np.array_equal(got[0], alone[i][0])
