@@ -1138,12 +1138,12 @@ AngWorkspace &ang_ws(int device) {
   return *p;
 }
 
-// Bytes a launch's workspace may take: a quarter of what is free or held by it.
-// (A quarter of what is free beside all that is held would rise from call to
-// call: freeing 70 GB and allocating a little more took a call on 114,000 nodes
-// from 0.06 to 5 s, every time.)
+// Bytes a launch's workspace may take: half of what is free or held by it. (A
+// share of what is free beside all that is held would rise from call to call:
+// freeing 70 GB and allocating a little more took a call on 114,000 nodes from
+// 0.06 to 5 s, every time.)
 size_t ang_budget(const AngWorkspace &w, size_t free_b) {
-  return (free_b + w.lane_bytes + w.wave_bytes) / 4;
+  return (free_b + w.lane_bytes + w.wave_bytes) / 2;
 }
 
 // Grows the workspace to the plan (lane maps of per_wave lanes per wave,
@@ -1280,6 +1280,32 @@ uint32_t sources_per_wave(uint32_t n_real, uint32_t simds) {
   return std::max<uint32_t>(1, std::min<uint32_t>(kWave, per));
 }
 
+// A launch's first sizes. Sources search with the bucket queue first; one that
+// overfills a bucket (or whose graph's costs leave the ring) runs again with
+// the heap.
+static AngPlan first_plan(uint32_t N, uint32_t maxp) {
+  AngPlan p;
+  p.maxp = maxp;
+  const uint32_t cap0 = default_tuning().cap;  // search states per lane before a retry
+  p.scap = std::min<uint32_t>(2 * N, cap0 ? std::max<uint32_t>(cap0, 2) : 8192u);
+  p.ncap = std::min<uint32_t>(N, p.scap);
+  p.hcap = 2 * p.scap;
+  p.bq_cap = bucket_capacity();
+  return p;
+}
+
+uint32_t angular_lanes(uint32_t N, uint32_t T, uint32_t maxp, uint32_t n, int dev) {
+  AngPlan p = first_plan(N, maxp);
+  int n_cu = 0;
+  hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev), "attribute");
+  p.per_wave = sources_per_wave(n, 4u * (uint32_t)n_cu);
+  ang_layout(p, N, T);
+  size_t total = 0;
+  hip_check(hipDeviceTotalMem(&total, dev), "total memory");
+  const size_t waves = total / 2 / (p.lane_stride * p.per_wave + p.wave_stride);
+  return (uint32_t)std::min<size_t>(n, std::max<size_t>(waves, 1) * p.per_wave);
+}
+
 void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items,
                           uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress) {
   if (specs.empty()) return;
@@ -1287,14 +1313,12 @@ void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<u
   int n_cu = 0;
   hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev0), "attribute");
   if ((explicit_items ? explicit_items->size() : n_implicit) == 0) return;
-  // one wave per source with its search in LDS; what does not fit there (or a
-  // launch it does not take) searches with one lane per source below
-  bool done = false;
+  // one wave per source with its search in LDS where that pays; what does not
+  // fit there, and what it does not take, searches with one lane per source below
   std::vector<uint2> rest;
-  if (!default_tuning().ang_lanes) rest = launch_simplest_wave(specs, explicit_items, n_implicit, stream, st, progress, &done);
-  if (done) {
+  if (!default_tuning().ang_lanes &&
+      launch_simplest_wave(specs, explicit_items, n_implicit, stream, st, progress, &rest)) {
     if (rest.empty()) return;
-    st.retries += (uint32_t)rest.size();
     explicit_items = &rest;
   }
   const uint32_t n_real = explicit_items ? (uint32_t)explicit_items->size() : n_implicit;
@@ -1342,15 +1366,7 @@ void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<u
     j.tstride = sp.tstride ? sp.tstride : sp.cs.T;
     j.reach = sp.d_reach;
   }
-  AngPlan p;
-  p.maxp = maxp;
-  const uint32_t cap0 = default_tuning().cap;  // search states per lane before a retry
-  p.scap = std::min<uint32_t>(2 * N, cap0 ? std::max<uint32_t>(cap0, 2) : 8192u);
-  p.ncap = std::min<uint32_t>(N, p.scap);
-  p.hcap = 2 * p.scap;
-  // sources search with the bucket queue first; one that overfills a bucket
-  // (or whose graph's costs leave the ring) runs again with the heap
-  p.bq_cap = bucket_capacity();
+  AngPlan p = first_plan(N, maxp);
   const int dev = specs[0].dg->device;
   hipDeviceProp_t prop;
   hip_check(hipGetDeviceProperties(&prop, dev), "props");

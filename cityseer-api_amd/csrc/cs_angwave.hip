@@ -1075,6 +1075,24 @@ AngWaveGraph &wave_graph(Graph &g, DevEdges &de) {
     to_device(perm, &w->perm);
     to_device(orig, &w->orig);
   }
+  if (ok) {
+    // A search's time per reached node, which hangs on how many states settle
+    // together. The smallest increment out of any state of the front bounds that:
+    // its likely size is what two in a hundred states lie below. Measured on
+    // duals of lattices with their nodes moved by up to 20, 8, 3, 1 and 0.3 m and
+    // of streets cut into pieces (300 sources, about 1,000 nodes each), that
+    // increment over the largest and the time: 4e-3 0.96 us, 1.8e-3 1.14, 7.6e-4
+    // 1.34, 2.7e-4 2.15, 8.4e-5 3.5, 5e-7 3.1 to 4.2.
+    std::vector<float> out;
+    for (const float x : wm)
+      if (std::isfinite(x)) out.push_back(x);
+    float low = 0.0f;
+    if (!out.empty() && w->max_w > 0.0f) {
+      std::nth_element(out.begin(), out.begin() + out.size() / 50, out.end());
+      low = out[out.size() / 50] / w->max_w;
+    }
+    w->state_ms = 0.95e-3f * std::clamp(std::pow(4e-3f / std::max(low, 1e-9f), 0.3f), 1.0f, 4.4f);
+  }
   w->usable = ok;
   de.ang_wave = std::move(w);
   return *de.ang_wave;
@@ -1128,6 +1146,7 @@ const AngWaveGraph::Reach &wave_reach(Graph &g, const DevEdges &de, AngWaveGraph
     std::sort(pg.begin(), pg.end());
     inner += (uint64_t)(std::unique(pg.begin(), pg.end()) - pg.begin());
   }
+  r.mean = (float)all / (float)kProbes;
   r.chains = (double)inner > 0.75 * (double)all;
   if (w.reach.size() >= 64) w.reach.clear();
   return w.reach[maxsec] = r;
@@ -1193,66 +1212,187 @@ void release_angular_wave_workspaces() {
   }
 }
 
-std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items,
-                                        uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress,
-                                        bool *done) {
-  *done = false;
-  const int dev = specs[0].dg->device;
-  // (also guards what the device's graphs keep for this search: a served slice
-  // comes without the graph's own lock)
-  WaveWorkspace &ws = wave_ws(dev);
-  std::lock_guard<std::mutex> lk(ws.mu);
-  const uint32_t cap = default_tuning().cap;
+namespace {
+
+// Requests whose searches run in one launch, laid out for the largest of them.
+struct WaveClass {
+  std::vector<uint32_t> specs;  // of the caller's
+  uint32_t n = 0;               // searches
   uint32_t N = 1, T = 1, maxp = 1, nodes = 0;
   uint32_t pages[10] = {0};
-  size_t rows = 0;
-  bool chains = false;
-  for (const AngSpec &sp : specs) {
-    if (sp.cs.betweenness && sp.cs.tolerance > kTieEps) return {};  // predecessors rebuilt from final routes (Phase 2)
-    if (!(sp.cs.maxsec >= 0.0f)) return {};
-    AngWaveGraph &w = wave_graph(*sp.g, *sp.de);
-    if (!w.usable) return {};
-    const AngWaveGraph::Reach &r = wave_reach(*sp.g, *sp.de, w, sp.cs.maxsec);
-    N = std::max(N, sp.g->n);
-    T = std::max(T, sp.cs.T);
-    maxp = std::max(maxp, sp.g->max_in_deg);
-    nodes = std::max(nodes, r.nodes);
-    chains = chains || r.chains;
-    for (uint32_t ps = kPage; ps < 10; ++ps) pages[ps] = std::max(pages[ps], r.pages[ps]);
-    rows += (size_t)4 * sp.cs.T * sp.g->n;
-  }
+  bool chains = false, betw = false;
+  double mean = 0.0, visits = 0.0;  // nodes of a search (the most over the requests), of all searches
+  double most = 0.0, all = 0.0;     // search time of the slowest request's sources, of all sources (ms)
+  double lane = 0.0;                // a lane's time per node (lane_cost)
+  uint32_t lds = 0;                 // 0: does not fit
   WaveArgs a;
-  std::memset(&a, 0, sizeof(a));
-  uint32_t lds = 0;
+  double ms = 0.0;
+};
+
+// Expected time of a launch, n searches on the waves that its LDS leaves room
+// for. Beside the time per node a search has a fixed part that grows with the
+// waves a CU runs (its results' atomics): 0.045 ms alone, 0.165 at twelve. On
+// the 150x150 lattice's dual, all 32,549 sources, expected and measured ms:
+// 400 m 2.1, 2.1; 800 m 3.4, 3.1; 2,000 m 17.4, 17.0; 3,200 m 104, 109.
+void wave_cost(WaveClass &c, uint32_t cap, uint32_t cus) {
+  std::memset(&c.a, 0, sizeof(c.a));
+  // a search settles up to two states a node (1.8 where it reaches thousands):
+  // past the positions that a state word holds most would fail
+  if (2.0 * c.mean > kMaxStates || !wave_layout(c.a, c.N, c.nodes, c.pages, 1.0, cap, c.chains, &c.lds)) {
+    c.lds = 0;
+    c.ms = INFINITY;
+    return;
+  }
+  const double W = std::min<double>(c.n, (double)cus * std::min(12u, kLdsMax / c.lds));
+  const double fixed = 0.045 + 0.01 * std::max(0.0, W / cus - 1.0);
+  c.ms = std::max(fixed + c.most, (c.n * fixed + c.all) / W) + 0.15;
+}
+
+// Expected time of a lane-per-source launch. At 100 sources and a reach of 1,000
+// a lane's search takes `per` us a node (0.64 of it without betweenness), a
+// little more the farther it reaches, and with 32,768 sources 3.6 (2.8) times
+// that; from there on more sources take in proportion longer. Measured on the
+// same dual to 2,000 m (and on one of 20 m pieces to 800 m): 100 sources 14.5
+// (11.3) us, 2,000 27.6 (22), 8,000 38 (27.5), 32,549 (30,000) 52.5 (38.8),
+// 113,865 (109,880) 139 (115); all sources to 400 m 37, to 3,200 m 58 (to 200 m 32).
+double lane_cost(uint32_t n, uint32_t lanes, double per, double mean, double visits, bool betw) {
+  const double m = std::min(std::min<double>(n, lanes), 32768.0), k = std::max(m, 100.0) / 100.0;
+  const double t = 1e-3 * per * std::pow(std::max(mean, 30.0) / 1000.0, 0.1) * (betw ? std::pow(k, 0.22) : 0.64 * std::pow(k, 0.255));
+  return 0.35 + t * std::max(mean, visits / m);
+}
+
+void merge(WaveClass &c, const WaveClass &d) {
+  c.specs.insert(c.specs.end(), d.specs.begin(), d.specs.end());
+  c.n += d.n;
+  c.N = std::max(c.N, d.N);
+  c.T = std::max(c.T, d.T);
+  c.maxp = std::max(c.maxp, d.maxp);
+  c.nodes = std::max(c.nodes, d.nodes);
+  for (int k = 0; k < 10; ++k) c.pages[k] = std::max(c.pages[k], d.pages[k]);
+  c.chains = c.chains || d.chains;
+  c.betw = c.betw || d.betw;
+  c.mean = std::max(c.mean, d.mean);
+  c.visits += d.visits;
+  c.most = std::max(c.most, d.most);
+  c.all += d.all;
+  c.lane = std::max(c.lane, d.lane);
+}
+
+// The requests that search in LDS, by launch; the others are the lanes' (their
+// numbers in `lanes`). A wave per source is the faster search until many sources
+// have to take turns: the 150x150 lattice's dual to 3,200 m (three waves a CU,
+// 32,549 sources) 109 ms against 145 with a lane per source, but a dual of 20 m
+// pieces to 1,600 m (one wave a CU) 18 against 47 with 100 sources, 125 against
+// 86 with 2,000 and 471 against 108 with 8,000. And a lane launch lasts as long
+// as its slowest source, so what it can take along is cheap there.
+std::vector<WaveClass> wave_plan(const std::vector<AngSpec> &specs, const std::vector<uint32_t> &count, uint32_t cap,
+                                 uint32_t cus, std::vector<uint32_t> *lanes) {
+  std::vector<WaveClass> cls;
+  WaveClass rest;  // the lanes' part
+  for (uint32_t i = 0; i < specs.size(); ++i) {
+    const AngSpec &sp = specs[i];
+    if (!count[i]) continue;
+    // (a larger tolerance rebuilds its predecessors from final routes, Phase 2)
+    const bool takes = !(sp.cs.betweenness && sp.cs.tolerance > kTieEps) && sp.cs.maxsec >= 0.0f &&
+                       wave_graph(*sp.g, *sp.de).usable;
+    WaveClass c;
+    c.specs = {i};
+    c.n = count[i];
+    c.N = sp.g->n;
+    c.T = sp.cs.T;
+    c.maxp = std::max(1u, sp.g->max_in_deg);
+    c.betw = sp.cs.betweenness;
+    c.lane = 14.7;
+    if (takes) {
+      AngWaveGraph &w = *sp.de->ang_wave;
+      const AngWaveGraph::Reach &r = wave_reach(*sp.g, *sp.de, w, sp.cs.maxsec);
+      c.nodes = r.nodes;
+      c.mean = r.mean;
+      c.chains = r.chains;
+      for (uint32_t ps = kPage; ps < 10; ++ps) c.pages[ps] = r.pages[ps];
+      c.visits = (double)c.n * r.mean;
+      c.most = (double)w.state_ms * r.mean;
+      c.all = c.n * c.most;
+      if (w.state_ms > 2e-3f) c.lane = 11.1;  // (as on the pieces)
+      wave_cost(c, cap, cus);
+    }
+    if (!takes || !c.lds) merge(rest, c);
+    else cls.push_back(std::move(c));
+  }
+  // neighbours in size share a launch where that is the faster
+  std::sort(cls.begin(), cls.end(), [](const WaveClass &x, const WaveClass &y) { return x.nodes < y.nodes; });
+  while (cls.size() > 1) {
+    double best = 0.0;
+    size_t at = cls.size();
+    WaveClass both;
+    for (size_t k = 0; k + 1 < cls.size(); ++k) {
+      WaveClass m = cls[k];
+      merge(m, cls[k + 1]);
+      wave_cost(m, cap, cus);
+      if (m.lds && cls[k].ms + cls[k + 1].ms - m.ms > best) {
+        best = cls[k].ms + cls[k + 1].ms - m.ms;
+        at = k;
+        both = std::move(m);
+      }
+    }
+    if (at == cls.size()) break;
+    cls[at] = std::move(both);
+    cls.erase(cls.begin() + at + 1);
+  }
+  // what a lane launch does sooner goes there, the slowest first
+  std::sort(cls.begin(), cls.end(), [](const WaveClass &x, const WaveClass &y) { return x.ms > y.ms; });
+  auto lane_ms = [&](const WaveClass &c) {
+    return c.n ? lane_cost(c.n, angular_lanes(c.N, c.T, c.maxp, c.n, specs[0].dg->device), c.lane, c.mean, c.visits, c.betw) : 0.0;
+  };
+  double now = lane_ms(rest);
+  for (size_t k = 0; k < cls.size();) {
+    WaveClass m = rest;
+    merge(m, cls[k]);
+    const double with = lane_ms(m);
+    if (with - now < cls[k].ms) {
+      rest = std::move(m);
+      now = with;
+      cls.erase(cls.begin() + k);
+    } else {
+      ++k;
+    }
+  }
+  *lanes = rest.specs;
+  return cls;
+}
+
+// One launch (two, where some of its sources outgrow their room): `items`
+// {request of the caller's, source position}, empty for all n of the one
+// request. What is left over goes to rest.
+void run_class(WaveWorkspace &ws, WaveClass &c, const std::vector<AngSpec> &specs, std::vector<uint2> items, uint32_t cap,
+               uint32_t cus, hipStream_t stream, cs_stats &st, uint32_t *progress, std::vector<uint2> *rest) {
+  WaveArgs a = c.a;
+  uint32_t lds = c.lds;
   // a little room beyond the probed sources, and more where that costs no
   // resident wave of the launch
-  if (!wave_layout(a, N, nodes, pages, 1.0, cap, chains, &lds)) return {};
   double room = 1.0;
-  hipDeviceProp_t prop;
-  hip_check(hipGetDeviceProperties(&prop, dev), "props");
-  const uint32_t cus = (uint32_t)prop.multiProcessorCount;
-  const uint32_t want = std::min<uint32_t>(explicit_items ? (uint32_t)explicit_items->size() : n_implicit, cus * (kLdsMax / lds));
+  const uint32_t want = std::min<uint32_t>(c.n, cus * (kLdsMax / lds));
   for (double f : {1.02, 1.05, 1.1, 1.2, 1.5, 2.0}) {
     WaveArgs b = a;
     uint32_t bl = 0;
-    if (!wave_layout(b, N, nodes, pages, f, cap, chains, &bl) || cus * (kLdsMax / bl) < want) break;
+    if (!wave_layout(b, c.N, c.nodes, c.pages, f, cap, c.chains, &bl) || cus * (kLdsMax / bl) < want) break;
     a = b;
     lds = bl;
     room = f;
   }
   static_assert(sizeof(WaveJob) % 4 == 0, "job table");
-  std::vector<uint2> items;
-  if (explicit_items) items = *explicit_items;
-  uint32_t n_list = explicit_items ? (uint32_t)items.size() : n_implicit;
+  uint32_t n_list = c.n;
   if (!ws.e0) {
     hip_check(hipEventCreate(&ws.e0), "event");
     hip_check(hipEventCreate(&ws.e1), "event");
   }
+  size_t rows = 0;
+  for (const uint32_t i : c.specs) rows += (size_t)4 * specs[i].cs.T * specs[i].g->n;
   double *acc = static_cast<double *>(ws.acc.get(8 * rows, "angular result rows"));
   hip_check(hipMemsetAsync(acc, 0, 8 * rows, stream), "memset");
-  std::vector<WaveJob> jobs(specs.size());
+  std::vector<WaveJob> jobs(specs.size());  // (of the class's requests)
   size_t at = 0;
-  for (size_t i = 0; i < specs.size(); ++i) {
+  for (const uint32_t i : c.specs) {
     const AngSpec &sp = specs[i];
     const AngWaveGraph &w = *sp.de->ang_wave;
     WaveJob &j = jobs[i];
@@ -1285,7 +1425,6 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
   char *ctl = static_cast<char *>(ws.ctl.get(256, "control words"));
   hip_check(hipMemsetAsync(ctl + 128, 0, 32, stream), "memset stats");
   uint32_t *d_fail = static_cast<uint32_t *>(ws.fail.get(4ull * n_list, "failure list"));
-  *done = true;
   for (int tier = 0; tier < 2; ++tier) {
     a.jobs = d_jobs;
     a.items = nullptr;
@@ -1296,7 +1435,7 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
       a.items = d_items;
     }
     a.n_items = n_list;
-    a.maxp = maxp;
+    a.maxp = c.maxp;
     // scratch of a wave: records | seconds | far list | page numbers | inner numbers |
     // seeds | predecessor lists | push seconds | node bests | path counts
     const size_t slots = (size_t)a.P << kPage;
@@ -1310,8 +1449,8 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
     a.o_far = take(2ull * a.F);
     a.o_pl = take(4ull * a.P);
     a.o_iid = take(2ull * a.S);
-    a.o_seed = take(8ull * T * a.S);
-    a.o_ext = take(4 * slots * (maxp + 1));
+    a.o_seed = take(8ull * c.T * a.S);
+    a.o_ext = take(4 * slots * (c.maxp + 1));
     a.o_psec = take(8 * slots);
     a.o_best = take(8 * slots);
     a.o_sig = take(8ull * a.S);
@@ -1358,21 +1497,22 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
     n_list = n_failed;
     unsigned long long stv[4];
     std::memcpy(stv, hctl + 32, 32);
-    if (tier == 1 || n_failed == 0 || cap) {
+    st.retries += n_failed;
+    // (no second try where a source may settle as many states as there can be)
+    if (tier == 1 || n_failed == 0 || cap || a.S == kMaxStates) {
       st.nodes_reached += stv[0];
       st.edges_scanned += stv[1];
       st.within_sum += stv[2];
       break;
     }
     // the rest once more with as much room as one workgroup per CU has
-    st.retries += n_failed;
     double wider = room;
     WaveArgs wide = a;
     uint32_t wide_lds = lds;
     for (double f = room * 1.25; f < 40.0; f *= 1.2) {
       WaveArgs b = a;
       uint32_t bl = 0;
-      if (!wave_layout(b, N, nodes, pages, f, 0, true, &bl)) break;
+      if (!wave_layout(b, c.N, c.nodes, c.pages, f, 0, true, &bl)) break;
       wide = b;
       wide_lds = bl;
       wider = f;
@@ -1388,16 +1528,49 @@ std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const
     a = wide;
     lds = wide_lds;
   }
-  for (size_t i = 0; i < specs.size(); ++i) {
+  for (const uint32_t i : c.specs) {
     const WaveJob &j = jobs[i];
     const size_t n = (size_t)4 * j.T * j.N;
     hipLaunchKernelGGL(k_wave_rows, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, stream, specs[i].d_acc, j.acc,
                        j.orig, j.N, j.T, specs[i].tstride ? specs[i].tstride : specs[i].cs.T);
   }
   hip_check(hipGetLastError(), "k_wave_rows launch");
-  // the staging belongs to the next call once the lock is released
+  // the staging belongs to the next launch, or the next call once the lock is released
   hip_check(hipStreamSynchronize(stream), "sync");
-  return items;
+  rest->insert(rest->end(), items.begin(), items.end());
+}
+
+}  // namespace
+
+bool launch_simplest_wave(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items, uint32_t n_implicit,
+                          hipStream_t stream, cs_stats &st, uint32_t *progress, std::vector<uint2> *rest) {
+  const int dev = specs[0].dg->device;
+  // (also guards what the device's graphs keep for this search: a served slice
+  // comes without the graph's own lock)
+  WaveWorkspace &ws = wave_ws(dev);
+  std::lock_guard<std::mutex> lk(ws.mu);
+  int n_cu = 0;
+  hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev), "attribute");
+  const uint32_t cap = default_tuning().cap, cus = (uint32_t)n_cu;
+  std::vector<uint32_t> count(specs.size(), 0), lanes;
+  if (explicit_items)
+    for (const uint2 &x : *explicit_items) ++count[x.x];
+  else
+    count[0] = n_implicit;
+  std::vector<WaveClass> cls = wave_plan(specs, count, cap, cus, &lanes);
+  if (cls.empty()) return false;
+  auto of = [&](const std::vector<uint32_t> &which) {  // the items of some requests, in the caller's order
+    std::vector<uint8_t> in(specs.size(), 0);
+    for (const uint32_t i : which) in[i] = 1;
+    std::vector<uint2> out;
+    for (const uint2 &x : *explicit_items)
+      if (in[x.x]) out.push_back(x);
+    return out;
+  };
+  if (explicit_items && !lanes.empty()) *rest = of(lanes);
+  for (WaveClass &c : cls)
+    run_class(ws, c, specs, explicit_items ? of(c.specs) : std::vector<uint2>(), cap, cus, stream, st, progress, rest);
+  return true;
 }
 
 }  // namespace cs

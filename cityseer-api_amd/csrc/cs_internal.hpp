@@ -80,10 +80,12 @@ struct AngWaveGraph {
   float *wm = nullptr;
   uint32_t *perm = nullptr, *orig = nullptr;
   float max_w = 0.0f;
+  float state_ms = 0.0f;  // a search's time per reached node (wave_graph)
   // nodes and runs of 2^k nodes (k < 10) that searches up to a time limit reach:
   // the most over a few probed sources, per limit asked for so far
   struct Reach {
     uint32_t nodes = 0;
+    float mean = 0.0f;  // nodes, the mean over the probed sources
     uint32_t pages[10] = {0};
     bool chains = false;  // most nodes lead on to others (streets cut into short pieces)
   };
@@ -452,11 +454,14 @@ void launch_simplest_jobs(const std::vector<AngSpec> &specs, const std::vector<u
                           uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress = nullptr);
 
 // The same with each source's whole search in the LDS of one wave
-// (cs_angwave.hip), where every request allows it (`done` false: none ran).
-// Returns the items whose search did not fit, which have added nothing.
-std::vector<uint2> launch_simplest_wave(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items,
-                                        uint32_t n_implicit, hipStream_t stream, cs_stats &st, uint32_t *progress,
-                                        bool *done);
+// (cs_angwave.hip), for the requests that allow it and where it is the faster
+// search. False when none is (nothing ran); else the items left over, which
+// have added nothing, are in rest.
+bool launch_simplest_wave(const std::vector<AngSpec> &specs, const std::vector<uint2> *explicit_items, uint32_t n_implicit,
+                          hipStream_t stream, cs_stats &st, uint32_t *progress, std::vector<uint2> *rest);
+// Lanes of n sources that a lane-per-source launch over graphs of up to N nodes
+// runs at once, as far as half of the device's memory holds them.
+uint32_t angular_lanes(uint32_t N, uint32_t T, uint32_t maxp, uint32_t n, int dev);
 void release_angular_wave_workspaces();
 
 void launch_simplest(Graph &g, DevGraph &dg, DevEdges &de, const CallSpec &cs,

@@ -3,7 +3,8 @@ everywhere (one at a time, and many at one route), streets cut into short straig
 states safe together), crossings of more than four streets (longer rows than one state's lanes),
 more thresholds than one back-propagation pass holds, and searches that outgrow the room the
 probed sources asked for (a dense knot in a sparse network; many dense cores, where searches run out
-of pages at a run of nodes met for the first time and their waves go on to other sources)."""
+of pages at a run of nodes met for the first time and their waves go on to other sources). And which
+calls that search takes: it and one lane per source give the same results."""
 
 from __future__ import annotations
 
@@ -13,6 +14,7 @@ import numpy as np
 import pytest
 
 from cityseer import _native
+from cityseer.serving import CentralityServer
 from cityseer.tools import mock
 import oracle.oracle as O
 from oracle.oracle import OracleGraph
@@ -105,6 +107,52 @@ def test_waves_search_on_after_running_out_of_pages():
     ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest([1200], n_threads=8)
     assert np.array_equal(got[0], ref[0])
     assert_close(got, ref, "dense cores")
+
+
+def _pieces(side, seed):
+    """A dual of streets cut into 20 m pieces, where nearly every state settles alone."""
+    return mock.network_structure_from_lattice(
+        mock.lattice_dual(mock.decompose_lattice(mock.perturbed_lattice(side, seed=seed), 20.0)))
+
+
+@pytest.mark.parametrize("side,distances,n_src,in_lds", [
+    (22, [900], 60, True),      # few long searches: a wave each
+    (22, [1800], 5254, False),  # many: they would take turns, a lane each does not
+    (40, [2600], 12, False),    # more states than a state word has positions for
+])
+def test_which_search(side, distances, n_src, in_lds):
+    O.set_heap_mode(False)
+    ns = _pieces(side, seed=75)
+    src = np.linspace(0, ns.node_count() - 1, n_src).astype(int).tolist()
+    say(f"{ns.node_count()} dual nodes in 20 m pieces, {n_src} sources, {distances} m")
+    got = stack(ns.centrality_simplest(distances=distances, source_indices=src), SIMPLEST, distances)
+    assert _native.last_lds_searches() == (n_src if in_lds else 0)
+    plan = ns._sampling_plan(None, None, None, src)
+    ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest(
+        distances, sources=plan["sources"], eligible=plan["eligible"], scale=plan["scale"], n_threads=8)
+    assert np.array_equal(got[0], ref[0])
+    assert_close(got, ref, "pieces")
+
+
+def test_requests_of_all_sizes_served_together():
+    """Served slices whose requests go to several launches in LDS, to lanes, and to both."""
+    nets = [mock.network_structure_from_lattice(mock.lattice_dual(x)) for x in
+            (mock.perturbed_lattice(50, seed=76), _star(9, 3, 1.0), _cores(40, 2, 9))] + [_pieces(22, seed=77)]
+    some = np.linspace(0, nets[3].node_count() - 1, 5000).astype(int).tolist()
+    mix = [(nets[0], dict(distances=[400])), (nets[3], dict(distances=[1800], source_indices=some)),
+           (nets[1], dict(distances=[250, 600])), (nets[2], dict(distances=[300, 900])),
+           (nets[3], dict(distances=[300], source_indices=some[::100])), (nets[0], dict(distances=[700, 1500])),
+           (nets[2], dict(distances=[500], compute_betweenness=False)),
+           (nets[1], dict(distances=[400], tolerance=0.03))]
+    alone = [ns.centrality_simplest(**kw) for ns, kw in mix]
+    say(f"{len(mix)} simplest requests at once")
+    with CentralityServer(slice_ms=50.0) as srv:
+        reqs = [srv.submit_simplest(ns, **kw) for ns, kw in mix]
+        for k, ((ns, kw), r, want) in enumerate(zip(mix, reqs, alone)):
+            r.wait()
+            x, y = (stack(v, SIMPLEST, kw["distances"]) for v in (r.result(), want))
+            assert np.array_equal(x[0], y[0]), f"request {k}"
+            assert_close(x, y, f"request {k}")
 
 
 def test_lane_workspace_does_not_creep():
