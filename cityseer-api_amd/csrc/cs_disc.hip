@@ -887,7 +887,9 @@ __global__ void k_disc_rows(const uint4 *rows, const uint2 *rev, const uint2 *fw
   for (uint32_t k = n; k < blocks * kQuad; ++k) out[k] = make_uint4(kNoNb, kInf, kInf, 0u);
 }
 
-constexpr uint32_t kProbes = 8, kProbeList = 65536, kProbeStop = 40000, kProbeWords = 16;
+// Probed sources: eight spread over the node order and one in its middle, which
+// on the Hilbert curve of a town as wide as its searches is the town's.
+constexpr uint32_t kProbes = 9, kProbeList = 65536, kProbeStop = 40000, kProbeWords = 16;
 constexpr uint32_t kProbePages = 10;  // page shifts of a probe's table: 4 .. 9
 
 struct ProbeArgs {
@@ -915,7 +917,8 @@ __global__ __launch_bounds__(512) void k_disc_probe(ProbeArgs a) {
   constexpr uint32_t kBands = 32;
   __shared__ uint32_t n_seen, n_next, n_far, kept, inner, pages[kProbePages];
   const uint32_t tid = threadIdx.x, B = blockDim.x;
-  const uint32_t src = (uint32_t)(((uint64_t)2 * blockIdx.x + 1) * a.N / (2 * kProbes));
+  const uint32_t src = blockIdx.x + 1 == kProbes ? a.N / 2
+                                                 : (uint32_t)(((uint64_t)2 * blockIdx.x + 1) * a.N / (2 * (kProbes - 1)));
   uint32_t *secs = a.secs + (size_t)blockIdx.x * a.N;
   uint32_t *mark = a.mark + (size_t)blockIdx.x * (a.N + a.pages), *pmark = mark + a.N;
   uint32_t *seen = a.lists + (size_t)blockIdx.x * 5 * a.cap;
@@ -1229,19 +1232,28 @@ static bool disc_takes(const JobSpec &js, DevVec &tmp, hipStream_t stream) {
 }
 
 // Is a workgroup per source, at `lds` bytes each, the faster search? Its rate
-// falls with the workgroups a CU holds; a wave per source with its state in
-// scratch holds twenty a CU whatever the reach, and takes five times as long
-// for each. Both measured on one 37,370-node network of streets in 20 m
-// pieces, kernel ms here | there, 7,474 sources:
-//   closeness, 5 workgroups (reach 3,607)  1.71 | 2.71,  3 (5,456)  3.14 | 3.95,  2 (7,566)  5.42 | 5.31,  1 (12,345)  14.6 | 10.8
-//   betweenness, 4 (3,607)  3.73 | 4.75,  3 (4,495)  5.51 | 5.76,  2 (5,456)  8.87 | 6.87,  1 (12,345)  34.9 | 19.2
-// and with few sources (reach 12,380, 1 workgroup a CU):
-//   224: closeness 0.60 | 4.63, betweenness 1.65 | 7.07;  1,023: 2.23 | 4.85, 5.52 | 7.87;  2,047: 4.25 | 5.38, 9.95 | 9.12
-// (reach 7,500, 2 a CU):
-//   224: 0.41 | 1.48, 0.84 | 2.22;  1,023: 0.86 | 1.55, 3.04 | 2.54;  2,989: 2.34 | 2.37, 6.27 | 4.14
+// falls with the waves its workgroups put on a CU; a wave per source with its
+// state in scratch has twenty a CU whatever the reach. Both measured, kernel ms
+// here | there (L: 300x300 lattice, P: 39,000 nodes in 20 m pieces, both with
+// workgroups of four waves).
+// Betweenness, 16 waves a CU:
+//   L reach 5,027: 1,600 sources 1.75 | 2.82,  6,400 5.49 | 7.54,  70,000 54.4 | 61.4
+// 12 waves:
+//   L 6,480: 1,600 2.79 | 3.65,  3,200 4.74 | 5.03,  6,400 8.63 | 9.71,  70,000 87.6 | 79.3
+//   P 5,035: 3,200 2.85 | 3.06,  6,400 5.26 | 5.91,  12,000 9.45 | 9.79
+// 8 waves:
+//   L 8,090: 800 2.39 | 3.71,  1,600 4.29 | 4.58,  3,200 7.69 | 6.26
+//   P 6,150: 800 1.44 | 1.86,  1,600 2.53 | 2.37,  3,200 4.48 | 3.69
+// 4 waves:
+//   P 11,400: 300 2.08 | 2.98,  800 3.94 | 3.39,  1,600 7.16 | 4.31
+// Closeness, 8 waves:
+//   L 9,830: 1,600 1.55 | 2.53,  70,000 51.3 | 59.4;  P 8,620: 3,200 2.71 | 2.82,  12,000 9.35 | 8.98
+// 4 waves:
+//   P 14,380: 800 2.10 | 2.09,  1,600 3.64 | 3.11,  3,200 6.77 | 4.58
 static bool disc_pays(uint32_t lds, uint32_t waves, bool betw, uint32_t n, uint32_t cus) {
-  const uint32_t per_cu = blocks_by_lds(lds);
-  return per_cu * waves >= (betw ? 12u : 8u) || n <= cus * per_cu * (betw ? 1u : 4u);
+  const uint32_t per_cu = blocks_by_lds(lds) * waves;
+  if (!betw) return per_cu >= 8 || n <= 4 * cus;
+  return per_cu >= 16 || n <= (per_cu >= 12 ? 28 : per_cu >= 8 ? 5 : 2) * cus;
 }
 
 // Splits the jobs' items into launches; what cannot search in LDS goes to rest.

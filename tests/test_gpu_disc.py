@@ -1,7 +1,8 @@
 """GPU: the LDS shortest search where it could go wrong, against the oracle: exact ties everywhere,
 rows of one to four blocks and beyond, one-way and parallel edges, streets cut into short pieces, a
 single very short edge (nodes that settle alone), either result by itself, more thresholds than one
-variant's registers, source subsets, and searches that outgrow the room the probed sources asked for."""
+variant's registers, source subsets, and searches that outgrow the room the probed sources asked for. And which
+calls that search takes."""
 
 from __future__ import annotations
 
@@ -89,6 +90,29 @@ def test_matches_oracle(name, distances, kw):
     assert in_lds == (0 if name == "star18" else stats["sources"])
     if name == "knot":
         assert stats["retries"] > 0
+
+
+@pytest.mark.parametrize("n_src,closeness,betweenness,in_lds", [
+    (300, True, True, True),     # one source a workgroup at once
+    (1600, True, True, False),   # dependencies of 6,000 nodes leave two workgroups a CU: they would take turns
+    (1600, True, False, True),   # without them the turns are short
+])
+def test_which_search(n_src, closeness, betweenness, in_lds):
+    O.set_heap_mode(False)
+    ns = mock.network_structure_from_lattice(mock.perturbed_lattice(110, seed=88))
+    src = np.linspace(0, ns.node_count() - 1, n_src).astype(int).tolist()
+    say(f"shortest search to 7,200 m, {n_src} sources, betweenness {betweenness}")
+    res = ns.centrality_shortest(distances=[800, 7200], source_indices=src, compute_closeness=closeness,
+                                 compute_betweenness=betweenness)
+    assert _native.last_lds_searches() == (n_src if in_lds else 0)
+    assert _native.last_stats()["retries"] == 0
+    plan = ns._sampling_plan(None, None, None, src)
+    ref, _ = OracleGraph.from_network_structure(ns).centrality_shortest(
+        [800, 7200], closeness=closeness, betweenness=betweenness, sources=plan["sources"], eligible=plan["eligible"],
+        scale=plan["scale"], n_threads=8)
+    got = stack(res, SHORTEST_KEYS, [800, 7200])
+    assert np.array_equal(got[0], ref[0])
+    assert_close(got, ref, "which search")
 
 
 def test_large_reach_is_searched_once():
