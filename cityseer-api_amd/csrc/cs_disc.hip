@@ -1199,6 +1199,8 @@ struct DiscClass {
   uint32_t lds = 0, waves = 1, NT = 1, N = 0;
   bool betw = false;
   double room = 1.0;
+  double most = 0.0, all = 0.0;  // expected time of its slowest search, of all its searches one by one (ms)
+  double load = 0.0;             // `all` on the workgroups the device holds
   DiscGraph::Reach reach;  // the most over its jobs
   std::vector<DiscJob> jobs;
   std::vector<uint32_t> which;  // the caller's job of each
@@ -1256,14 +1258,80 @@ static bool disc_pays(uint32_t lds, uint32_t waves, bool betw, uint32_t n, uint3
   return per_cu >= 16 || n <= (per_cu >= 12 ? 28 : per_cu >= 8 ? 5 : 2) * cus;
 }
 
+// Lays a launch out and estimates it: 0.05 ms and 0.17 us a node for a search
+// (0.06 us without betweenness; the 250x250 lattice to 5,000 m, 38 searches after
+// one another on five workgroups a CU: 25.7 and 8.6 ms), twenty waves a CU at
+// most. False when the layout does not fit.
+static bool disc_estimate(DiscClass &d, uint32_t cap, uint32_t cus) {
+  DiscArgs a;
+  std::memset(&a, 0, sizeof(a));
+  if (!disc_layout(a, d.N, d.reach, d.betw, d.waves, 1.0, cap, &d.lds)) return false;
+  d.load = d.all / ((double)cus * std::max(1u, std::min(blocks_by_lds(d.lds), 20u / d.waves)));
+  return true;
+}
+
+// Two launches as one, without their jobs.
+static DiscClass disc_pair(const DiscClass &x, const DiscClass &y) {
+  DiscClass d;
+  std::memset(&d.a, 0, sizeof(d.a));
+  d.NT = x.NT;
+  d.N = std::max(x.N, y.N);
+  d.n = x.n + y.n;
+  d.betw = x.betw || y.betw;
+  d.reach.nodes = std::max(x.reach.nodes, y.reach.nodes);
+  d.reach.front = std::max(x.reach.front, y.reach.front);
+  d.reach.inner = std::max(x.reach.inner, y.reach.inner);
+  for (int p = 0; p < 10; ++p) d.reach.pages[p] = std::max(x.reach.pages[p], y.reach.pages[p]);
+  d.a.maxp = std::max(x.a.maxp, y.a.maxp);
+  d.waves = std::max(x.waves, y.waves);
+  d.most = std::max(x.most, y.most);
+  d.all = x.all + y.all;
+  return d;
+}
+
+// Expected time of a launch: of its slowest search, or of its load with the
+// device running empty at its end.
+static double disc_time(const DiscClass &d) { return std::max(d.most, d.load + 0.5 * d.most); }
+
+// Joins launches, neighbours in size, while that shortens their time after one
+// another.
+static void disc_join(std::vector<DiscClass> &v, uint32_t cap, uint32_t cus) {
+  std::sort(v.begin(), v.end(), [](const DiscClass &x, const DiscClass &y) { return x.lds < y.lds; });
+  // what joining each with its next saves
+  std::vector<double> saves;
+  auto saved = [&](size_t k) {
+    DiscClass m = disc_pair(v[k], v[k + 1]);
+    return disc_estimate(m, cap, cus) ? disc_time(v[k]) + disc_time(v[k + 1]) - disc_time(m) : -INFINITY;
+  };
+  for (size_t k = 0; k + 1 < v.size(); ++k) saves.push_back(saved(k));
+  while (v.size() > 1) {
+    const size_t k = (size_t)(std::max_element(saves.begin(), saves.end()) - saves.begin());
+    if (!(saves[k] > 0.0)) break;
+    DiscClass m = disc_pair(v[k], v[k + 1]);
+    (void)disc_estimate(m, cap, cus);
+    for (DiscClass *x : {&v[k], &v[k + 1]}) {
+      m.which.insert(m.which.end(), x->which.begin(), x->which.end());
+      m.jobs.insert(m.jobs.end(), x->jobs.begin(), x->jobs.end());
+    }
+    v[k] = std::move(m);
+    v.erase(v.begin() + k + 1);
+    saves.erase(saves.begin() + k);
+    if (k < saves.size()) saves[k] = saved(k);
+    if (k) saves[k - 1] = saved(k - 1);
+  }
+}
+
 // Splits the jobs' items into launches; what cannot search in LDS goes to rest.
+// A launch is laid out for its largest search, so jobs share one where their
+// sizes are alike or all their sources run at once anyway: seven towns of 9x9 to
+// 28x28 to 1,200 m 0.50 ms as seven launches after one another, 0.24 with a wave
+// per source in one launch.
 static std::vector<DiscClass> disc_plan(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, DevVec &tmp,
                                         hipStream_t stream, std::vector<uint2> *rest) {
   std::vector<DiscClass> out;
-  std::vector<int> cls(specs.size(), -1);
-  std::vector<uint32_t> local(specs.size(), 0);
-  int cus = 0;
-  hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, specs[0].dg->device), "attribute");
+  int n_cu = 0;
+  hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, specs[0].dg->device), "attribute");
+  const uint32_t cus = (uint32_t)n_cu;
   for (size_t i = 0; i < specs.size(); ++i) {
     const JobSpec &js = specs[i];
     std::lock_guard<std::mutex> lk(js.de->disc_mu);
@@ -1279,34 +1347,24 @@ static std::vector<DiscClass> disc_plan(const std::vector<JobSpec> &specs, uint3
     for (uint32_t ps = 4; ps < kProbePages; ++ps) r.pages[ps] = (js.g->n + (1u << ps) - 1) >> ps;
     uint32_t waves = disc_waves((uint32_t)(2.0 * std::sqrt((double)js.g->n)));
     if (!disc_layout(a, js.g->n, r, js.cs.betweenness, waves, 1.0, cap, &lds) ||
-        js.n_sources > (uint32_t)cus * blocks_by_lds(lds)) {
+        js.n_sources > cus * blocks_by_lds(lds)) {
       r = disc_reach(*js.g, w, js.cs.maxsec, tmp, stream);
       waves = disc_waves(r.front);
       if (!disc_layout(a, js.g->n, r, js.cs.betweenness, waves, 1.0, cap, &lds)) continue;
     }
-    if (!disc_pays(lds, waves, js.cs.betweenness, js.n_sources, (uint32_t)cus)) continue;
-    int c = -1;
-    for (size_t k = 0; k < out.size(); ++k)
-      if (out[k].waves == waves && out[k].betw == js.cs.betweenness && lds * 4 <= out[k].lds * 5 && out[k].lds * 4 <= lds * 5)
-        c = (int)k;
-    if (c < 0) {
-      c = (int)out.size();
-      out.emplace_back();
-      out[c].waves = waves;
-      out[c].NT = NT;
-      out[c].betw = js.cs.betweenness;
-      out[c].lds = lds;
-    }
-    DiscClass &d = out[c];
-    cls[i] = c;
-    local[i] = (uint32_t)d.jobs.size();
+    if (!disc_pays(lds, waves, js.cs.betweenness, js.n_sources, cus)) continue;
+    DiscClass d;
+    std::memset(&d.a, 0, sizeof(d.a));
+    d.waves = waves;
+    d.NT = NT;
+    d.betw = js.cs.betweenness;
     d.which.push_back((uint32_t)i);
-    d.N = std::max(d.N, js.g->n);
-    d.reach.nodes = std::max(d.reach.nodes, r.nodes);
-    d.reach.front = std::max(d.reach.front, r.front);
-    d.reach.inner = std::max(d.reach.inner, r.inner);
-    for (int p = 0; p < 10; ++p) d.reach.pages[p] = std::max(d.reach.pages[p], r.pages[p]);
-    d.a.maxp = std::max(d.a.maxp, std::max(1u, w.maxp));
+    d.N = js.g->n;
+    d.n = js.n_sources;
+    d.reach = r;
+    d.a.maxp = std::max(1u, w.maxp);
+    d.most = 0.05 + (d.betw ? 1.7e-4 : 6e-5) * r.nodes;
+    d.all = d.n * d.most;
     DiscJob j;
     std::memset(&j, 0, sizeof(j));
     j.row = w.row;
@@ -1331,19 +1389,29 @@ static std::vector<DiscClass> disc_plan(const std::vector<JobSpec> &specs, uint3
       j.beta[t] = t < js.cs.T ? js.cs.beta[t] : 0.0f;
     }
     d.jobs.push_back(j);
+    if (disc_estimate(d, cap, cus)) out.push_back(std::move(d));
   }
   if (out.empty()) return out;
+  disc_join(out, cap, cus);
+  // (jobs that paid for their few sources alone may be many together)
+  out.erase(std::remove_if(out.begin(), out.end(),
+                           [&](const DiscClass &d) { return !disc_pays(d.lds, d.waves, d.betw, d.n, cus); }),
+            out.end());
+  if (out.empty()) return out;
   // items in the callers' order; one whole job alone needs no list
-  if (specs.size() == 1) {
-    out[0].n = specs[0].n_sources;
-  } else {
-    for (uint32_t i = 0; i < specs.size(); ++i)
-      for (uint32_t k = 0; k < specs[i].n_sources; ++k) {
-        if (cls[i] < 0) rest->push_back(make_uint2(i, k));
-        else out[cls[i]].items.push_back(make_uint2(local[i], k));
-      }
-    for (DiscClass &d : out) d.n = (uint32_t)d.items.size();
-  }
+  if (specs.size() == 1) return out;
+  std::vector<int> cls(specs.size(), -1);
+  std::vector<uint32_t> local(specs.size(), 0);
+  for (size_t c = 0; c < out.size(); ++c)
+    for (size_t k = 0; k < out[c].which.size(); ++k) {
+      cls[out[c].which[k]] = (int)c;
+      local[out[c].which[k]] = (uint32_t)k;
+    }
+  for (uint32_t i = 0; i < specs.size(); ++i)
+    for (uint32_t k = 0; k < specs[i].n_sources; ++k) {
+      if (cls[i] < 0) rest->push_back(make_uint2(i, k));
+      else out[cls[i]].items.push_back(make_uint2(local[i], k));
+    }
   return out;
 }
 
@@ -1396,6 +1464,14 @@ static bool disc_shape(DiscClass &d, uint32_t cap, int dev, bool first, uint32_t
   return true;
 }
 
+// A launch's 256 bytes of control words, zero when it starts.
+static void disc_ctl(DiscArgs &a, char *ctl) {
+  a.stats = reinterpret_cast<unsigned long long *>(ctl + 128);
+  a.next = reinterpret_cast<uint32_t *>(ctl);
+  a.n_fail = a.next + kXcd;
+  a.fail_flags = a.next + kXcd + 1;
+}
+
 static void disc_args(DiscClass &d, char *ctl, uint32_t *fail, const uint2 *items, const DiscJob *jobs, char *scratch,
                       uint32_t *progress, uint32_t blocks) {
   DiscArgs &a = d.a;
@@ -1403,17 +1479,13 @@ static void disc_args(DiscClass &d, char *ctl, uint32_t *fail, const uint2 *item
   a.items = d.items.empty() ? nullptr : items;
   a.n_items = d.n;
   a.ws = scratch;
-  a.stats = reinterpret_cast<unsigned long long *>(ctl + 128);
-  a.next = reinterpret_cast<uint32_t *>(ctl);
-  a.n_fail = a.next + kXcd;
-  a.fail_flags = a.next + kXcd + 1;
+  disc_ctl(a, ctl);
   a.fail_list = fail;
   for (uint32_t x = 0; x <= kXcd; ++x) a.xbeg[x] = (uint32_t)((uint64_t)d.n * x / kXcd);
   a.progress = progress_room(progress, blocks);
 }
 
-static void disc_enqueue(const DiscClass &d, uint32_t blocks, char *ctl, hipStream_t stream) {
-  hipLaunchKernelGGL(k_disc_zero, dim3(1), dim3(kWave), 0, stream, reinterpret_cast<uint64_t *>(ctl), 32u);
+static void disc_enqueue(const DiscClass &d, uint32_t blocks, hipStream_t stream) {
   const dim3 grid(blocks), block(d.waves * kWave);
   if (d.NT <= 1) hipLaunchKernelGGL(k_disc<1>, grid, block, d.lds, stream, d.a);
   else if (d.NT <= 2) hipLaunchKernelGGL(k_disc<2>, grid, block, d.lds, stream, d.a);
@@ -1461,7 +1533,8 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
     uint32_t *fail_list = static_cast<uint32_t *>(ws->fail.get(4ull * d.n, "failure list"));
     disc_args(d, ctl, fail_list, items, jobs, scratch, progress, blocks);
     hip_check(hipEventRecord(ws->e0, stream), "event");
-    disc_enqueue(d, blocks, ctl, stream);
+    hipLaunchKernelGGL(k_disc_zero, dim3(1), dim3(kWave), 0, stream, reinterpret_cast<uint64_t *>(ctl), 32u);
+    disc_enqueue(d, blocks, stream);
     hip_check(hipGetLastError(), "k_disc launch");
     hip_check(hipEventRecord(ws->e1, stream), "event");
     uint32_t h[64];
@@ -1506,17 +1579,18 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
 }
 
 // The launches of a fixed set of jobs, for a batch that replays them from a
-// graph: memory of their own, nothing of it changed between runs.
+// graph: memory of their own, nothing of it changed between runs. They follow
+// one another: beside one another on four branches of the graph a replay was 3
+// to 20% shorter, but each branch has a stream of its own made first, and a
+// batch's first run took 1 to 5 ms more.
 struct DiscBatch {
   struct Part {
     DiscClass d;
     uint32_t blocks = 0;
-    char *ctl = nullptr;
     uint32_t *fail = nullptr;
   };
   std::vector<Part> parts;
   std::vector<void *> bufs;
-  char *ctl = nullptr;  // [parts][256]
   uint32_t waves = 0;
   ~DiscBatch() {
     for (void *q : bufs) (void)hipFree(q);
@@ -1557,11 +1631,8 @@ DiscBatch *disc_batch_new(const std::vector<JobSpec> &specs, uint32_t NT, int de
     b->parts.push_back(std::move(p));
   }
   if (b->parts.empty()) return nullptr;
-  char *ws = static_cast<char *>(b->mem(scratch));  // (the launches follow one another)
-  b->ctl = static_cast<char *>(b->mem(256 * b->parts.size()));
-  for (size_t i = 0; i < b->parts.size(); ++i) {
-    DiscBatch::Part &p = b->parts[i];
-    p.ctl = b->ctl + 256 * i;
+  char *ws = static_cast<char *>(b->mem(scratch));
+  for (DiscBatch::Part &p : b->parts) {
     p.fail = static_cast<uint32_t *>(b->mem(4ull * p.d.n));
     DiscJob *jobs = static_cast<DiscJob *>(b->mem(sizeof(DiscJob) * p.d.jobs.size()));
     hip_check(hipMemcpy(jobs, p.d.jobs.data(), sizeof(DiscJob) * p.d.jobs.size(), hipMemcpyHostToDevice), "copy");
@@ -1570,25 +1641,28 @@ DiscBatch *disc_batch_new(const std::vector<JobSpec> &specs, uint32_t NT, int de
       items = static_cast<uint2 *>(b->mem(sizeof(uint2) * p.d.n));
       hip_check(hipMemcpy(items, p.d.items.data(), sizeof(uint2) * p.d.n, hipMemcpyHostToDevice), "copy");
     }
-    disc_args(p.d, p.ctl, p.fail, items, jobs, ws, nullptr, p.blocks);
+    disc_args(p.d, nullptr, p.fail, items, jobs, ws, nullptr, p.blocks);
   }
   return b.release();
 }
 
 void disc_batch_delete(DiscBatch *b) { delete b; }
 
-void disc_batch_enqueue(const DiscBatch &b, hipStream_t stream) {
-  for (const DiscBatch::Part &p : b.parts) disc_enqueue(p.d, p.blocks, p.ctl, stream);
+size_t disc_batch_ctl(const DiscBatch &b) { return 256 * b.parts.size(); }
+
+void disc_batch_enqueue(DiscBatch &b, char *ctl, hipStream_t stream) {
+  for (size_t i = 0; i < b.parts.size(); ++i) {
+    disc_ctl(b.parts[i].d.a, ctl + 256 * i);
+    disc_enqueue(b.parts[i].d, b.parts[i].blocks, stream);
+  }
 }
 
-void disc_batch_collect(const DiscBatch &b, hipStream_t stream, cs_stats &st, std::vector<uint2> *retry) {
-  std::vector<uint32_t> h(64 * b.parts.size());
-  hip_check(hipMemcpyAsync(h.data(), b.ctl, 4 * h.size(), hipMemcpyDeviceToHost, stream), "copy");
-  hip_check(hipStreamSynchronize(stream), "sync");
+void disc_batch_collect(const DiscBatch &b, const char *ctl, cs_stats &st, std::vector<uint2> *retry) {
   st.waves = std::max(st.waves, b.waves);
   for (size_t i = 0; i < b.parts.size(); ++i) {
     const DiscBatch::Part &p = b.parts[i];
-    const uint32_t *c = &h[64 * i];
+    uint32_t c[64];
+    std::memcpy(c, ctl + 256 * i, 256);
     unsigned long long stv[4];
     std::memcpy(stv, c + 32, 32);
     st.nodes_reached += stv[0];

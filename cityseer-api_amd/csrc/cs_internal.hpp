@@ -324,14 +324,16 @@ struct JobSpec {
 bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, hipStream_t stream, cs_stats &st,
                  uint32_t *progress, std::vector<uint2> *rest);
 // The same for a fixed set of jobs run many times: prepared once (null: none
-// can), enqueued (under capture too), and its counts and the items that ran out
-// of room taken after each run.
+// can; rest: what it leaves), enqueued under capture, and its counts and the items
+// that ran out of room taken from a copy of its control words after each run. ctl:
+// disc_batch_ctl bytes, zero when a run starts.
 struct DiscBatch;
 DiscBatch *disc_batch_new(const std::vector<JobSpec> &specs, uint32_t NT, int device, hipStream_t stream,
                           std::vector<uint2> *rest);
 void disc_batch_delete(DiscBatch *b);
-void disc_batch_enqueue(const DiscBatch &b, hipStream_t stream);
-void disc_batch_collect(const DiscBatch &b, hipStream_t stream, cs_stats &st, std::vector<uint2> *retry);
+size_t disc_batch_ctl(const DiscBatch &b);
+void disc_batch_enqueue(DiscBatch &b, char *ctl, hipStream_t stream);
+void disc_batch_collect(const DiscBatch &b, const char *ctl, cs_stats &st, std::vector<uint2> *retry);
 // Nodes of a search up to maxsec as far as probed searches tell, with a quarter
 // more (0: none were).
 uint32_t disc_nodes(const DevEdges &de, float maxsec);

@@ -2277,8 +2277,10 @@ struct ShortestBatch {
   std::vector<uint2> items;
   Job *d_jobs = nullptr;
   uint2 *d_items = nullptr;
+  // control words: 64 bytes of the search in scratch, its statistics, the others'
+  static constexpr size_t kCtl = 128;
+  size_t ctl_bytes = kCtl;
   uint32_t *d_ctl = nullptr, *d_fail = nullptr;
-  unsigned long long *d_stats = nullptr;
   Workspace ws;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -2290,12 +2292,11 @@ struct ShortestBatch {
     if (graph) (void)hipGraphDestroy(graph);
     exec = nullptr;
     graph = nullptr;
-    for (void *q : {(void *)d_jobs, (void *)d_items, (void *)d_ctl, (void *)d_fail, (void *)d_stats})
+    for (void *q : {(void *)d_jobs, (void *)d_items, (void *)d_ctl, (void *)d_fail})
       if (q) (void)hipFree(q);
     d_jobs = nullptr;
     d_items = nullptr;
     d_ctl = d_fail = nullptr;
-    d_stats = nullptr;
     disc_batch_delete(disc);
     disc = nullptr;
     ws.release();
@@ -2354,8 +2355,8 @@ struct ShortestBatch {
     hip_check(hipMalloc(&d_items, sizeof(uint2) * std::max<uint64_t>(n_items, 1)), "hipMalloc items");
     if (!items.empty())
       hip_check(hipMemcpy(d_items, items.data(), sizeof(uint2) * items.size(), hipMemcpyHostToDevice), "copy");
-    hip_check(hipMalloc(&d_ctl, 64), "hipMalloc ctl");
-    hip_check(hipMalloc(&d_stats, 32), "hipMalloc stats");
+    ctl_bytes = kCtl + (disc ? disc_batch_ctl(*disc) : 0);
+    hip_check(hipMalloc(&d_ctl, ctl_bytes), "hipMalloc ctl");
     hip_check(hipMalloc(&d_fail, 4 * std::max<uint64_t>(n_items, 1)), "hipMalloc fail");
     ws.device = device;
     if (n_items) prepare_ws(ws, maxN, p.stride, waves, 0, stream);
@@ -2363,13 +2364,12 @@ struct ShortestBatch {
     // capture: clear control words, statistics and accumulators, then search
     SearchArgs a = args();
     hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "begin capture");
-    hipLaunchKernelGGL(k_zero64, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint64_t *>(d_ctl), (size_t)8);
-    hipLaunchKernelGGL(k_zero64, dim3(1), dim3(64), 0, stream, reinterpret_cast<uint64_t *>(d_stats), (size_t)4);
+    hipLaunchKernelGGL(k_zero64, dim3(1), dim3(256), 0, stream, reinterpret_cast<uint64_t *>(d_ctl), ctl_bytes / 8);
     for (const ZeroRegion &z : zero) {
       const size_t grid = std::min<size_t>((z.words + 255) / 256, 4096);
       if (z.words) hipLaunchKernelGGL(k_zero64, dim3((uint32_t)grid), dim3(256), 0, stream, z.ptr, z.words);
     }
-    if (disc) disc_batch_enqueue(*disc, stream);
+    if (disc) disc_batch_enqueue(*disc, reinterpret_cast<char *>(d_ctl) + kCtl, stream);
     if (n_items) launch_nt<kBrandes>(NT, waves / wpb, block, lds, stream, a);
     hipError_t le = hipGetLastError();
     hipError_t ce = hipStreamEndCapture(stream, &graph);
@@ -2388,7 +2388,7 @@ struct ShortestBatch {
     a.bcap = p.bcap;
     a.cap = p.cap;
     a.nbk_lds = p.nbk;
-    a.stats = d_stats;
+    a.stats = reinterpret_cast<unsigned long long *>(d_ctl + 16);
     a.keys = ws.keys;
     a.ncap = ws.ncap;
     a.ws = static_cast<char *>(ws.scratch.p);
@@ -2429,11 +2429,11 @@ struct ShortestBatch {
     hip_check(hipEventRecord(e0, stream), "event record");
     hip_check(hipGraphLaunch(exec, stream), "graph launch");
     hip_check(hipEventRecord(e1, stream), "event record");
-    uint32_t ctl[16];
+    std::vector<uint32_t> ctl(ctl_bytes / 4);
     unsigned long long stv[4];
-    hip_check(hipMemcpyAsync(ctl, d_ctl, 64, hipMemcpyDeviceToHost, stream), "copy ctl");
-    hip_check(hipMemcpyAsync(stv, d_stats, 32, hipMemcpyDeviceToHost, stream), "copy stats");
+    hip_check(hipMemcpyAsync(ctl.data(), d_ctl, ctl_bytes, hipMemcpyDeviceToHost, stream), "copy ctl");
     hip_check(hipStreamSynchronize(stream), "sync");
+    std::memcpy(stv, &ctl[16], 32);
     float ms = 0.0f;
     hip_check(hipEventElapsedTime(&ms, e0, e1), "elapsed");
     (void)hipEventDestroy(e0);
@@ -2444,7 +2444,7 @@ struct ShortestBatch {
     st.edges_scanned += stv[1];
     st.within_sum += stv[2];
     std::vector<uint2> retry;
-    if (disc) disc_batch_collect(*disc, stream, st, &retry);
+    if (disc) disc_batch_collect(*disc, reinterpret_cast<const char *>(ctl.data()) + kCtl, st, &retry);
     const uint32_t n_failed = ctl[kXcd], flags = ctl[kXcd + 1];
     if (n_failed == 0 && retry.empty()) return;
     if (flags & kFailWide) fail_wide_row();

@@ -21,10 +21,10 @@ from test_gpu_shortest import SHORTEST_KEYS, assert_close, say, stack
 pytestmark = pytest.mark.gpu
 
 
-def _knot():
-    """A lattice at 100 m with one 14 x 14 lattice at 4 m hung on its corner: the searches there reach
+def _knot(side=60, size=14):
+    """A lattice at 100 m with one size x size lattice at 4 m hung on its corner: the searches there reach
     many times as many nodes as the rest."""
-    a, b = mock.perturbed_lattice(60, seed=5), mock.perturbed_lattice(14, spacing=4.0, jitter=1.0, seed=6)
+    a, b = mock.perturbed_lattice(side, seed=5), mock.perturbed_lattice(size, spacing=4.0, jitter=1.0, seed=6)
     k = len(a.x)
     return mock.Lattice(x=np.concatenate([a.x, b.x + a.x[0] - 100.0]), y=np.concatenate([a.y, b.y + a.y[0] - 100.0]),
                         edges=np.concatenate([a.edges, b.edges + k, [[0, k]]]),
@@ -135,10 +135,12 @@ def test_large_reach_is_searched_once():
 
 
 def test_batch_mixes_searches_and_replays():
-    """One batch of searches in LDS, of two sizes, some out of room, and in scratch; every replay the same."""
+    """One batch of searches in LDS, of two sizes, some out of room, and in scratch; every replay the same.
+    (The knot is a twentieth of its network's node order, before its first probed source, and its 1,296
+    nodes are past 1.3 times the 400 or so that any probed source of the batch reaches.)"""
     nets = [mock.network_structure_from_lattice(x) for x in
-            (_knot(), _star(18, 3, 1.0), mock.perturbed_lattice(13, seed=82), mock.perturbed_lattice(50, seed=87))]
-    asked = [[150, 300], [300], [200, 500], [2500]]
+            (_knot(160, 36), _star(18, 3, 1.0), mock.perturbed_lattice(13, seed=82), mock.perturbed_lattice(50, seed=87))]
+    asked = [[150, 300], [300], [200, 500], [1500]]
     alone = [stack(ns.centrality_shortest(distances=d), SHORTEST_KEYS, d) for ns, d in zip(nets, asked)]
     with CentralityBatch() as batch:
         for ns, d in zip(nets, asked):
@@ -154,3 +156,20 @@ def test_batch_mixes_searches_and_replays():
                 assert np.array_equal(got[0], alone[i][0])
                 assert_close(got, alone[i], f"network {i}, run {k}")
             nets[2].centrality_shortest(distances=[400])
+
+
+def test_batch_of_small_towns_is_one_launch():
+    """Towns of very different sizes whose sources all run at once: a workgroup for each, in one launch."""
+    nets = [mock.network_structure_from_lattice(mock.perturbed_lattice(s, seed=90 + s)) for s in (9, 11, 13, 16, 19, 23, 28)]
+    alone = [stack(ns.centrality_shortest(distances=[400, 1200]), SHORTEST_KEYS, [400, 1200]) for ns in nets]
+    with CentralityBatch() as batch:
+        for ns in nets:
+            batch.add_shortest(ns, distances=[400, 1200])
+        for k in range(2):
+            say(f"batch of {len(nets)} small towns, run {k}")
+            stats = batch.run()
+            assert _native.last_lds_searches() == stats["sources"] and stats["waves"] >= stats["sources"]
+            for i, res in enumerate(batch.results()):
+                got = stack(res, SHORTEST_KEYS, [400, 1200])
+                assert np.array_equal(got[0], alone[i][0])
+                assert_close(got, alone[i], f"town {i}, run {k}")
