@@ -1505,6 +1505,14 @@ void run_class(WaveWorkspace &ws, WaveClass &c, const std::vector<AngSpec> &spec
       st.within_sum += stv[2];
       break;
     }
+    // (a few searched twice cost less than room for them in every wave)
+    if ((uint64_t)n_failed * 32 > c.n)
+      for (const uint32_t i : c.specs) {
+        const uint32_t n = specs[i].g->n;
+        AngWaveGraph::Reach &r = specs[i].de->ang_wave->reach[specs[i].cs.maxsec];
+        r.nodes = std::min(n, r.nodes + r.nodes / 4 + 1);
+        for (uint32_t ps = kPage; ps < 10; ++ps) r.pages[ps] = std::min((n >> ps) + 1, r.pages[ps] + r.pages[ps] / 4 + 1);
+      }
     // the rest once more with as much room as one workgroup per CU has
     double wider = room;
     WaveArgs wide = a;

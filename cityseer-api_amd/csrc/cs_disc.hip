@@ -1558,6 +1558,9 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
     std::vector<uint2> left(n_failed);
     for (uint32_t i = 0; i < n_failed; ++i) left[i] = d.items.empty() ? make_uint2(0u, fl[i]) : d.items[fl[i]];
     st.retries += n_failed;
+    // (a few searched twice cost less than room for them in every workgroup)
+    if (!cap && (uint64_t)n_failed * 32 > d.n)
+      for (const uint32_t i : d.which) (void)disc_more_room(*specs[i].de, specs[i].cs.maxsec, specs[i].g->n);
     // again with more room while LDS has it
     DiscClass e = d;
     e.items = left;
@@ -1679,6 +1682,23 @@ void disc_batch_collect(const DiscBatch &b, const char *ctl, cs_stats &st, std::
       retry->push_back(make_uint2(p.d.which[x.x], x.y));
     }
   }
+}
+
+bool disc_more_room(DevEdges &de, float maxsec, uint32_t N) {
+  std::lock_guard<std::mutex> lk(de.disc_mu);
+  if (!de.disc) return false;
+  const auto it = de.disc->reach.find(maxsec);
+  if (it == de.disc->reach.end()) return false;
+  DiscGraph::Reach &r = it->second;
+  bool more = false;
+  auto up = [&](uint32_t &x, uint32_t most) {
+    const uint32_t y = std::min(most, x + x / 4 + 1);
+    more = more || y > x;
+    x = std::max(x, y);
+  };
+  for (uint32_t *x : {&r.nodes, &r.front, &r.inner}) up(*x, N);
+  for (uint32_t ps = 4; ps < kProbePages; ++ps) up(r.pages[ps], (N + (1u << ps) - 1) >> ps);
+  return more;
 }
 
 uint32_t disc_nodes(const DevEdges &de, float maxsec) {

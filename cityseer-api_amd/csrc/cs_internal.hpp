@@ -334,6 +334,9 @@ void disc_batch_delete(DiscBatch *b);
 size_t disc_batch_ctl(const DiscBatch &b);
 void disc_batch_enqueue(DiscBatch &b, char *ctl, hipStream_t stream);
 void disc_batch_collect(const DiscBatch &b, const char *ctl, cs_stats &st, std::vector<uint2> *retry);
+// Searches up to maxsec outgrew the room that the probed ones asked for: a
+// quarter more from now on. False when there is no more to give.
+bool disc_more_room(DevEdges &de, float maxsec, uint32_t N);
 // Nodes of a search up to maxsec as far as probed searches tell, with a quarter
 // more (0: none were).
 uint32_t disc_nodes(const DevEdges &de, float maxsec);

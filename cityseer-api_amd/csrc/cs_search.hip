@@ -2451,6 +2451,15 @@ struct ShortestBatch {
     if (flags & kFailInternal) fail(CS_EINTERNAL, "search invariant violated (bucket order)");
     if (flags & kFailRing) fail(CS_EINTERNAL, "bucket ring window exceeded");
     st.retries += n_failed + (uint32_t)retry.size();
+    // searches out of room cost a replay a launch of their own: the next run
+    // plans with more (a quarter each time)
+    bool replan = false;
+    std::vector<uint8_t> seen(specs.size(), 0);
+    for (const uint2 &x : retry)
+      if (!seen[x.x]) {
+        seen[x.x] = 1;
+        replan = disc_more_room(*specs[x.x].de, specs[x.x].cs.maxsec, specs[x.x].g->n) || replan;
+      }
     Tuning t2 = tune;
     if (n_failed) {
       std::vector<uint32_t> fl(n_failed);
@@ -2460,6 +2469,7 @@ struct ShortestBatch {
       t2.cap = std::min<uint32_t>(std::max<uint32_t>(p.cap * 4, 4096), kSlotLimit);
     }
     run_jobs<kBrandes>(specs, NT, t2, nullptr, stream, st, &retry);
+    if (replan) ready = false;
   }
 
   // Times each candidate launch shape on every k-th source and keeps the

@@ -102,11 +102,15 @@ def test_waves_search_on_after_running_out_of_pages():
     O.set_heap_mode(False)
     ns = mock.network_structure_from_lattice(mock.lattice_dual(_cores(70, 4, 12)))
     say(f"angular search, dense cores: {ns.node_count()} dual nodes")
-    got = stack(ns.centrality_simplest(distances=[1200]), SIMPLEST, [1200])
-    assert _native.last_stats()["retries"] > 1000
     ref, _ = OracleGraph.from_network_structure(ns).centrality_simplest([1200], n_threads=8)
-    assert np.array_equal(got[0], ref[0])
-    assert_close(got, ref, "dense cores")
+    retries = []
+    for k in range(6):
+        got = stack(ns.centrality_simplest(distances=[1200]), SIMPLEST, [1200])
+        retries.append(_native.last_stats()["retries"])
+        assert np.array_equal(got[0], ref[0])
+        assert_close(got, ref, f"dense cores, call {k}")
+    assert retries[0] > 1000
+    assert retries[-1] * 32 <= ns.node_count(), retries  # (later calls have room for them)
 
 
 def _pieces(side, seed):

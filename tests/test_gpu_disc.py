@@ -173,3 +173,20 @@ def test_batch_of_small_towns_is_one_launch():
                 got = stack(res, SHORTEST_KEYS, [400, 1200])
                 assert np.array_equal(got[0], alone[i][0])
                 assert_close(got, alone[i], f"town {i}, run {k}")
+
+
+def test_batch_learns_the_room_its_searches_take():
+    """Runs of a batch whose knot outgrows the probed searches (1,296 nodes to their 75): each plans the next
+    with more room, until none searches twice; every run the same."""
+    ns = mock.network_structure_from_lattice(_knot(160, 36))
+    want = stack(ns.centrality_shortest(distances=[150, 300]), SHORTEST_KEYS, [150, 300])
+    with CentralityBatch() as batch:
+        batch.add_shortest(ns, distances=[150, 300])
+        retries = []
+        while not retries or retries[-1] > 0 and len(retries) < 24:
+            say(f"batch with a knot, run {len(retries)}")
+            retries.append(batch.run()["retries"])
+            got = stack(batch.results()[0], SHORTEST_KEYS, [150, 300])
+            assert np.array_equal(got[0], want[0])
+            assert_close(got, want, f"run {len(retries)}")
+    assert retries[0] > 0 and retries[-1] == 0, retries
