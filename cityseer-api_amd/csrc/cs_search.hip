@@ -2472,19 +2472,16 @@ struct ShortestBatch {
     if (replan) ready = false;
   }
 
-  // Times each candidate launch shape on every k-th source and keeps the
-  // fastest per source. The jobs' accumulators hold garbage afterwards; the
-  // next run clears them.
+  // Times each candidate launch shape on every k-th source that searches in
+  // scratch (the shapes are that search's; a batch without any keeps its own)
+  // and keeps the fastest per source. The jobs' accumulators hold garbage
+  // afterwards; the next run clears them.
   Tuning autotune(double fraction, hipStream_t stream) {
-    uint64_t total = 0;
-    for (auto &js : specs) total += js.n_sources;
-    if (total == 0) return tune;
+    if (!ready) prepare(stream);
+    if (n_items == 0) return tune;
     const uint64_t stride = std::max<uint64_t>(1, (uint64_t)std::llround(1.0 / std::max(fraction, 1e-6)));
     std::vector<uint2> sample;
-    uint64_t k = 0;
-    for (uint32_t jb = 0; jb < specs.size(); ++jb)
-      for (uint32_t i = 0; i < specs[jb].n_sources; ++i, ++k)
-        if (k % stride == 0) sample.push_back(make_uint2(jb, i));
+    for (uint64_t k = 0; k < n_items; k += stride) sample.push_back(items.empty() ? make_uint2(0u, (uint32_t)k) : items[k]);
     Tuning best = tune;
     double best_ms = INFINITY;
     for (uint32_t blk : {64u, 128u, 256u})

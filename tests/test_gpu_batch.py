@@ -10,6 +10,7 @@ from cityseer.batch import CentralityBatch
 from cityseer.tools import io, mock
 from oracle.oracle import OracleGraph
 import oracle.oracle as O
+from test_gpu_angular_wave import _star
 from test_gpu_shortest import assert_close, say, stack
 
 pytestmark = pytest.mark.gpu
@@ -93,6 +94,27 @@ def test_autotune_keeps_results(primal_graph):
     after = b.results()
     for (ns, kw), x, y in zip(reqs, before, after):
         _check_equal(y, x, kw["distances"], f"after autotune {tune}")
+
+
+def test_autotune_times_what_the_shapes_are_for():
+    """A launch shape is the search in scratch memory's: a batch that runs in LDS keeps its own, one with a
+    crossing of eighteen streets (rows too long for LDS) is tuned."""
+    ns = mock.network_structure_from_lattice(mock.perturbed_lattice(14, seed=3))
+    own = dict(block_threads=64, waves_per_simd=2, delta_scale=0.5, slot_capacity=0, xcd_split=True)
+    for nets in ([ns], [ns, mock.network_structure_from_lattice(_star(18, 3, 1.0))]):
+        b = CentralityBatch()
+        for x in nets:
+            b.add_shortest(x, distances=[300, 600])
+        b.set_tuning(**own)
+        say(f"autotune, {len(nets)} networks")
+        tune = b.autotune(0.5)
+        if len(nets) == 1:
+            assert {k: tune[k] for k in own} == {**own, "xcd_split": 1}
+        else:
+            assert tune["delta_scale"] in (0.75, 1.0)
+        b.run()
+        for x, r in zip(nets, b.results()):
+            _check_equal(r, x.centrality_shortest(distances=[300, 600]), [300, 600], f"after autotune {tune}")
 
 
 def test_explicit_tunings_agree():
