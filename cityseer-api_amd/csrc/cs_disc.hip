@@ -909,11 +909,12 @@ __global__ void k_fill32(uint32_t *p, size_t n, uint32_t v) {
 }
 
 // What a search takes, for a few sources spread over the node order, one a
-// workgroup: bands of seconds, within a band a node again whenever its seconds
+// workgroup, of each request (grid's y): bands of seconds, within a band a node again whenever its seconds
 // drop, lists in memory. Stops past what LDS holds. Each step is a round trip to
 // memory: 0.4 ms for a reach of 4,300 nodes (the same on the host from a copy of
 // the rows 3.8 ms).
-__global__ __launch_bounds__(512) void k_disc_probe(ProbeArgs a) {
+__global__ __launch_bounds__(512) void k_disc_probe(const ProbeArgs *args) {
+  const ProbeArgs a = args[blockIdx.y];
   constexpr uint32_t kBands = 32;
   __shared__ uint32_t n_seen, n_next, n_far, kept, inner, pages[kProbePages];
   const uint32_t tid = threadIdx.x, B = blockDim.x;
@@ -1035,76 +1036,133 @@ __global__ void k_disc_zero(uint64_t *p, uint32_t n) {
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// The graph's rows for this kernel, built once per speed, on the device from the
-// edge arrays it holds. They are there when this returns: another call may read
-// them on its own stream as soon as the caller lets go of disc_mu (a batch that
-// plans holds no other lock of the graph), and `tmp` may go to another call.
-DiscGraph &disc_graph(const Graph &g, const DevGraph &dg, DevEdges &de, DevVec &tmp, hipStream_t stream) {
-  if (de.disc) return *de.disc;
-  auto w = std::make_unique<DiscGraph>();
-  const uint32_t n = g.n, most = kMaxBlocks * kQuad;
-  if (n > 0 && n < (1u << 24) && !(de.min_es <= 0.0f) && g.max_out_deg <= most && g.max_in_deg <= most) {
-    constexpr uint32_t kInfo = 66;
-    const dim3 grid((n + 255) / 256), block(256);
-    uint64_t *info = static_cast<uint64_t *>(tmp.get(4ull * kInfo + 8ull * n, "row measures"));
-    uint2 *meas = reinterpret_cast<uint2 *>(info + kInfo / 2);
-    uint32_t h[kInfo];
-    hipLaunchKernelGGL(k_disc_zero, dim3(1), dim3(kWave), 0, stream, info, kInfo / 2);
-    hipLaunchKernelGGL(k_disc_measure, grid, block, 0, stream, dg.rows, de.rev_adj, de.fwd_adj, n, meas,
-                       reinterpret_cast<uint32_t *>(info));
-    hip_check(hipMemcpyAsync(h, info, sizeof(h), hipMemcpyDeviceToHost, stream), "copy");
-    hip_check(hipStreamSynchronize(stream), "sync");
-    w->blocks = std::max(1u, (h[0] + kQuad - 1) / kQuad);
-    w->maxp = std::max(1u, g.max_out_deg);
-    w->spans.assign(h + 2, h + kInfo);
-    w->usable = !h[1] && w->blocks <= kMaxBlocks;
-    if (w->usable) {
-      hip_check(hipMalloc(&w->row, sizeof(uint4) * n * w->blocks * kQuad), "hipMalloc rows");
-      hipLaunchKernelGGL(k_disc_rows, grid, block, 0, stream, dg.rows, de.rev_adj, de.fwd_adj, n, w->blocks, meas, w->row);
-      hip_check(hipGetLastError(), "rows launch");
-      hip_check(hipStreamSynchronize(stream), "sync");
+// The graphs' rows for this kernel, built once per speed, on the device from the
+// edge arrays they hold, all that are missing at once. They are there when this
+// returns: another call may read them on its own stream as soon as the caller
+// lets go of the graph's disc_mu, and `tmp` may go to another call.
+void disc_graphs(const std::vector<JobSpec> &specs, DevVec &tmp, hipStream_t stream) {
+  constexpr uint32_t kInfo = 66, most = kMaxBlocks * kQuad;
+  struct New {
+    const JobSpec *js;
+    std::unique_ptr<DiscGraph> w;
+    size_t meas;  // words from the start of tmp
+  };
+  std::vector<New> todo;
+  size_t words = 0;
+  for (const JobSpec &js : specs) {
+    const Graph &g = *js.g;
+    if (!js.n_sources || js.de->disc) continue;
+    bool there = false;
+    for (const New &x : todo) there = there || x.js->de == js.de;
+    if (there) continue;
+    if (!(g.n > 0 && g.n < (1u << 24) && !(js.de->min_es <= 0.0f) && g.max_out_deg <= most && g.max_in_deg <= most)) {
+      js.de->disc = std::make_unique<DiscGraph>();
+      continue;
     }
+    todo.push_back({&js, std::make_unique<DiscGraph>(), words});
+    words += 2 * (size_t)g.n;
   }
-  de.disc = std::move(w);
-  return *de.disc;
+  if (todo.empty()) return;
+  uint32_t *meas = static_cast<uint32_t *>(tmp.get(4 * (words + kInfo * todo.size()), "row measures")), *info = meas + words;
+  const dim3 block(256);
+  hipLaunchKernelGGL(k_fill32, dim3(1), block, 0, stream, info, kInfo * todo.size(), 0u);
+  for (size_t i = 0; i < todo.size(); ++i) {
+    const JobSpec &js = *todo[i].js;
+    hipLaunchKernelGGL(k_disc_measure, dim3((js.g->n + 255) / 256), block, 0, stream, js.dg->rows, js.de->rev_adj,
+                       js.de->fwd_adj, js.g->n, reinterpret_cast<uint2 *>(meas + todo[i].meas), info + kInfo * i);
+  }
+  hip_check(hipGetLastError(), "row measures launch");
+  std::vector<uint32_t> host(kInfo * todo.size());
+  hip_check(hipMemcpyAsync(host.data(), info, 4 * host.size(), hipMemcpyDeviceToHost, stream), "copy");
+  hip_check(hipStreamSynchronize(stream), "sync");
+  for (size_t i = 0; i < todo.size(); ++i) {
+    const JobSpec &js = *todo[i].js;
+    DiscGraph &w = *todo[i].w;
+    const uint32_t *h = &host[kInfo * i], n = js.g->n;
+    w.blocks = std::max(1u, (h[0] + kQuad - 1) / kQuad);
+    w.maxp = std::max(1u, js.g->max_out_deg);
+    w.spans.assign(h + 2, h + kInfo);
+    w.usable = !h[1] && w.blocks <= kMaxBlocks;
+    if (!w.usable) continue;
+    hip_check(hipMalloc(&w.row, sizeof(uint4) * n * w.blocks * kQuad), "hipMalloc rows");
+    hipLaunchKernelGGL(k_disc_rows, dim3((n + 255) / 256), block, 0, stream, js.dg->rows, js.de->rev_adj, js.de->fwd_adj, n,
+                       w.blocks, reinterpret_cast<const uint2 *>(meas + todo[i].meas), w.row);
+  }
+  hip_check(hipGetLastError(), "rows launch");
+  hip_check(hipStreamSynchronize(stream), "sync");
+  for (New &x : todo) x.js->de->disc = std::move(x.w);
 }
 
-// What searches up to maxsec take: the most over the probed sources.
-const DiscGraph::Reach &disc_reach(const Graph &g, DiscGraph &w, float maxsec, DevVec &tmp, hipStream_t stream) {
-  auto it = w.reach.find(maxsec);
-  if (it != w.reach.end()) return it->second;
-  const size_t n = g.n;
-  ProbeArgs a;
-  a.row = w.row;
-  a.N = g.n;
-  a.blocks = w.blocks;
-  a.maxsec = maxsec;
-  a.pages = 0;
-  for (uint32_t ps = 4; ps < kProbePages; ++ps) a.pages += (g.n >> ps) + 1;
-  a.cap = std::min(g.n, kProbeList);
-  const size_t words[] = {kProbes * n, kProbes * (n + a.pages), (size_t)kProbes * 5 * a.cap, kProbes * kProbeWords};
-  a.secs = static_cast<uint32_t *>(tmp.get(4 * (words[0] + words[1] + words[2] + words[3]), "probe scratch"));
-  a.mark = a.secs + words[0];
-  a.lists = a.mark + words[1];
-  a.out = a.lists + words[2];
-  hipLaunchKernelGGL(k_fill32, dim3(256), dim3(256), 0, stream, a.secs, words[0], kInf);
-  hipLaunchKernelGGL(k_fill32, dim3(256), dim3(256), 0, stream, a.mark, words[1], 0u);
-  hipLaunchKernelGGL(k_disc_probe, dim3(kProbes), dim3(512), 0, stream, a);
-  hip_check(hipGetLastError(), "probe launch");
-  uint32_t h[kProbes * kProbeWords];
-  hip_check(hipMemcpyAsync(h, a.out, sizeof(h), hipMemcpyDeviceToHost, stream), "copy");
-  hip_check(hipStreamSynchronize(stream), "sync");
-  DiscGraph::Reach r;
-  for (uint32_t k = 0; k < kProbes; ++k) {
-    const uint32_t *o = h + k * kProbeWords;
-    r.nodes = std::max(r.nodes, o[0]);
-    r.front = std::max(r.front, o[1]);
-    r.inner = std::max(r.inner, o[2]);
-    for (uint32_t ps = 4; ps < kProbePages; ++ps) r.pages[ps] = std::max(r.pages[ps], o[ps - 1]);
+// What the requests' searches take, the most over the probed sources of each, for
+// those not probed before: together, in as few launches as 256 MB of scratch
+// allow (a launch lasts as long as its longest chain of steps).
+void disc_probe(const std::vector<const JobSpec *> &asked, DevVec &tmp, hipStream_t stream) {
+  std::vector<const JobSpec *> todo;
+  for (const JobSpec *js : asked) {
+    bool there = js->de->disc->reach.count(js->cs.maxsec) != 0;
+    for (const JobSpec *x : todo) there = there || (x->de == js->de && x->cs.maxsec == js->cs.maxsec);
+    if (!there) todo.push_back(js);
+  }
+  auto pages_of = [](uint32_t n) {
+    uint32_t pages = 0;
+    for (uint32_t ps = 4; ps < kProbePages; ++ps) pages += (n >> ps) + 1;
+    return pages;
+  };
+  auto words_of = [&](uint32_t n) {
+    return (size_t)kProbes * (2 * (size_t)n + pages_of(n) + 5 * (size_t)std::min(n, kProbeList));
+  };
+  for (size_t i0 = 0; i0 < todo.size();) {
+    size_t i1 = i0, words = 0;
+    while (i1 < todo.size() && i1 - i0 < 4096 && (i1 == i0 || words + words_of(todo[i1]->g->n) <= (64u << 20))) words += words_of(todo[i1++]->g->n);
+    const size_t k = i1 - i0, table = (sizeof(ProbeArgs) * k + 3) / 4, out = k * kProbes * kProbeWords;
+    uint32_t *d = static_cast<uint32_t *>(tmp.get(4 * (table + out + words), "probe scratch"));
+    uint32_t *at = d + table + out;
+    std::vector<ProbeArgs> args(k);
+    size_t secs = 0, marks = 0;
+    for (size_t i = 0; i < k; ++i) secs += kProbes * (size_t)todo[i0 + i]->g->n;
+    for (size_t i = 0; i < k; ++i) marks += kProbes * (size_t)(todo[i0 + i]->g->n + pages_of(todo[i0 + i]->g->n));
+    size_t o_secs = 0, o_marks = secs, o_lists = secs + marks;
+    for (size_t i = 0; i < k; ++i) {
+      const JobSpec &js = *todo[i0 + i];
+      ProbeArgs &a = args[i];
+      a.row = js.de->disc->row;
+      a.N = js.g->n;
+      a.blocks = js.de->disc->blocks;
+      a.maxsec = js.cs.maxsec;
+      a.pages = pages_of(a.N);
+      a.cap = std::min(a.N, kProbeList);
+      a.secs = at + o_secs;
+      a.mark = at + o_marks;
+      a.lists = at + o_lists;
+      a.out = d + table + i * kProbes * kProbeWords;
+      o_secs += kProbes * (size_t)a.N;
+      o_marks += kProbes * (size_t)(a.N + a.pages);
+      o_lists += (size_t)kProbes * 5 * a.cap;
+    }
+    hip_check(hipMemcpyAsync(d, args.data(), sizeof(ProbeArgs) * k, hipMemcpyHostToDevice, stream), "copy");
+    hipLaunchKernelGGL(k_fill32, dim3(256), dim3(256), 0, stream, at, secs, kInf);
+    hipLaunchKernelGGL(k_fill32, dim3(256), dim3(256), 0, stream, at + secs, marks, 0u);
+    hipLaunchKernelGGL(k_disc_probe, dim3(kProbes, (uint32_t)k), dim3(512), 0, stream, reinterpret_cast<const ProbeArgs *>(d));
+    hip_check(hipGetLastError(), "probe launch");
+    std::vector<uint32_t> h(out);
+    hip_check(hipMemcpyAsync(h.data(), d + table, 4 * out, hipMemcpyDeviceToHost, stream), "copy");
+    hip_check(hipStreamSynchronize(stream), "sync");
+    for (size_t i = 0; i < k; ++i) {
+      DiscGraph::Reach r;
+      for (uint32_t q = 0; q < kProbes; ++q) {
+        const uint32_t *o = &h[(i * kProbes + q) * kProbeWords];
+        r.nodes = std::max(r.nodes, o[0]);
+        r.front = std::max(r.front, o[1]);
+        r.inner = std::max(r.inner, o[2]);
+        for (uint32_t ps = 4; ps < kProbePages; ++ps) r.pages[ps] = std::max(r.pages[ps], o[ps - 1]);
+      }
+      auto &known = todo[i0 + i]->de->disc->reach;
+      if (known.size() >= 64) known.clear();
+      known[todo[i0 + i]->cs.maxsec] = r;
+    }
+    i0 = i1;
   }
   if (tmp.bytes > (64u << 20)) tmp.release();
-  if (w.reach.size() >= 64) w.reach.clear();
-  return w.reach[maxsec] = r;
 }
 
 constexpr uint32_t kLdsMax = 159u * 1024u;  // (a workgroup's control words lie beside it)
@@ -1214,12 +1272,18 @@ struct DiscClass {
 // and 160, 3.44 at 24 and 48.
 static uint32_t disc_waves(uint32_t front) { return front <= 40 ? 1u : front <= 100 ? 2u : 4u; }
 
-// Can this request search in LDS (its other work is the caller's)?
-static bool disc_takes(const JobSpec &js, DevVec &tmp, hipStream_t stream) {
+// ... as far as the request itself tells.
+static bool disc_may(const JobSpec &js) {
   if (js.d_od_off || js.extra_records) return false;
   if (js.cs.betweenness && js.cs.tolerance > kTieEps) return false;  // predecessors rebuilt from final distances (Phase 2)
-  if (!(js.cs.maxsec >= 0.0f)) return false;
-  DiscGraph &w = disc_graph(*js.g, *js.dg, *js.de, tmp, stream);
+  return js.cs.maxsec >= 0.0f;
+}
+
+// Can this request search in LDS (its other work is the caller's)? Its graph's
+// rows are built.
+static bool disc_takes(const JobSpec &js) {
+  if (!disc_may(js)) return false;
+  const DiscGraph &w = *js.de->disc;
   if (!w.usable) return false;
   // where many nodes have an in-edge shorter than the tie bands at the search's
   // far end, they would settle one at a time
@@ -1332,23 +1396,54 @@ static std::vector<DiscClass> disc_plan(const std::vector<JobSpec> &specs, uint3
   int n_cu = 0;
   hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, specs[0].dg->device), "attribute");
   const uint32_t cus = (uint32_t)n_cu;
+  // what the graphs keep, in one order for all callers
+  std::vector<DevEdges *> des;
+  for (const JobSpec &js : specs) des.push_back(js.de);
+  std::sort(des.begin(), des.end(), std::less<DevEdges *>());
+  des.erase(std::unique(des.begin(), des.end()), des.end());
+  std::vector<std::unique_lock<std::mutex>> locks;
+  for (DevEdges *de : des) locks.emplace_back(de->disc_mu);
+  {
+    std::vector<JobSpec> may;
+    for (const JobSpec &js : specs)
+      if (disc_may(js)) may.push_back(js);
+    disc_graphs(may, tmp, stream);
+  }
+  struct Size {
+    bool takes = false, whole = false;
+    DiscGraph::Reach r;
+    uint32_t waves = 1, lds = 0;
+  };
+  std::vector<Size> sizes(specs.size());
+  std::vector<const JobSpec *> asked;
   for (size_t i = 0; i < specs.size(); ++i) {
     const JobSpec &js = specs[i];
-    std::lock_guard<std::mutex> lk(js.de->disc_mu);
-    if (!js.n_sources || !disc_takes(js, tmp, stream)) continue;
-    DiscGraph &w = *js.de->disc;
-    DiscArgs a;
-    std::memset(&a, 0, sizeof(a));
-    uint32_t lds = 0;
+    Size &z = sizes[i];
+    z.takes = js.n_sources && disc_takes(js);
+    if (!z.takes) continue;
     // a network so small that every source runs at once with room for all of
     // it needs no probes (they took a fifth of a first call on 676 nodes)
-    DiscGraph::Reach r;
-    r.nodes = r.front = r.inner = js.g->n;
-    for (uint32_t ps = 4; ps < kProbePages; ++ps) r.pages[ps] = (js.g->n + (1u << ps) - 1) >> ps;
-    uint32_t waves = disc_waves((uint32_t)(2.0 * std::sqrt((double)js.g->n)));
-    if (!disc_layout(a, js.g->n, r, js.cs.betweenness, waves, 1.0, cap, &lds) ||
-        js.n_sources > cus * blocks_by_lds(lds)) {
-      r = disc_reach(*js.g, w, js.cs.maxsec, tmp, stream);
+    DiscArgs a;
+    std::memset(&a, 0, sizeof(a));
+    z.r.nodes = z.r.front = z.r.inner = js.g->n;
+    for (uint32_t ps = 4; ps < kProbePages; ++ps) z.r.pages[ps] = (js.g->n + (1u << ps) - 1) >> ps;
+    z.waves = disc_waves((uint32_t)(2.0 * std::sqrt((double)js.g->n)));
+    z.whole = disc_layout(a, js.g->n, z.r, js.cs.betweenness, z.waves, 1.0, cap, &z.lds) &&
+              js.n_sources <= cus * blocks_by_lds(z.lds);
+    if (!z.whole) asked.push_back(&js);
+  }
+  disc_probe(asked, tmp, stream);
+  for (size_t i = 0; i < specs.size(); ++i) {
+    const JobSpec &js = specs[i];
+    if (!sizes[i].takes) continue;
+    DiscGraph &w = *js.de->disc;
+    DiscGraph::Reach &r = sizes[i].r;
+    uint32_t &waves = sizes[i].waves, &lds = sizes[i].lds;
+    if (!sizes[i].whole) {
+      DiscArgs a;
+      std::memset(&a, 0, sizeof(a));
+      if (!w.reach.count(js.cs.maxsec)) disc_probe({&js}, tmp, stream);  // (forgotten over more than 64 others)
+      r = w.reach.at(js.cs.maxsec);
       waves = disc_waves(r.front);
       if (!disc_layout(a, js.g->n, r, js.cs.betweenness, waves, 1.0, cap, &lds)) continue;
     }

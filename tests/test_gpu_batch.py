@@ -155,3 +155,17 @@ def test_batch_request_with_ten_thresholds():
     got = stack(res[1], KEYS, ten)
     assert np.array_equal(got[0], ref[0])
     assert_close(got, ref, "ten thresholds in a batch vs oracle")
+
+
+def test_batch_of_more_cutoffs_than_a_graph_keeps():
+    """Seventy requests of one network, each to its own distance: more probed searches than are remembered."""
+    ns = mock.network_structure_from_lattice(mock.perturbed_lattice(60, seed=22))
+    dists = [200 + 5 * k for k in range(70)]
+    b = CentralityBatch()
+    for d in dists:
+        b.add_shortest(ns, distances=[d])
+    say("seventy requests of one network")
+    b.run()
+    res = b.results()
+    for k in (0, 35, 69):
+        _check_equal(res[k], ns.centrality_shortest(distances=[dists[k]]), [dists[k]], f"request {k}")
