@@ -1531,11 +1531,14 @@ static bool disc_shape(DiscClass &d, uint32_t cap, int dev, bool first, uint32_t
   };
   if (!lay(d.room)) return false;
   if (first) {
+    // (steps of 1.08 from the probed sizes left a city without 0.7 ms for a few
+    // sources searched twice, or with them, as its probes fell)
     const uint32_t most = resident;
-    double room = d.room;
-    for (double r = d.room * 1.08; r < d.room * 2.0; r *= 1.08) {
-      if (!lay(r) || resident < most) break;
-      room = r;
+    double room = d.room, above = 2.0 * d.room;
+    for (double r = above; above - room > 0.015; r = 0.5 * (room + above)) {
+      if (lay(r) && resident == most) room = r;
+      else above = r;
+      if (room == above) break;
     }
     d.room = room;
     lay(room);

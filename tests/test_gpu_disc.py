@@ -115,6 +115,14 @@ def test_which_search(n_src, closeness, betweenness, in_lds):
     assert_close(got, ref, "which search")
 
 
+def test_city_is_searched_once():
+    """Room up to what costs no resident workgroup: no source of a large even network runs out of it."""
+    ns = mock.network_structure_from_lattice(mock.perturbed_lattice(200, seed=1, diag_frac=0.05))
+    say(f"shortest search, {ns.node_count()} nodes to 5,000 m")
+    ns.centrality_shortest(distances=[5000])
+    assert _native.last_stats()["retries"] == 0 and _native.last_lds_searches() == ns.node_count()
+
+
 def test_large_reach_is_searched_once():
     """Too large for a workgroup's LDS and for the usual records of a wave: no source is searched twice."""
     O.set_heap_mode(False)
