@@ -1,11 +1,14 @@
-"""Batched centrality: many shortest-path requests in one persistent GPU launch.
+"""Batched centrality: many shortest-path requests replayed as one graph of launches.
 
 A ``CentralityBatch`` collects ``node_centrality_shortest`` requests over any
 number of ``NetworkStructure`` graphs, each with its own thresholds, flags and
-sources, and runs all their sources in one persistent launch captured in a
-hipGraph (the first ``run`` captures it, later runs replay it). ``autotune``
-times candidate launch shapes (workgroup size, resident waves per SIMD, bucket
-width) on a sample of the batch's sources and keeps the fastest.
+sources. Searches that fit a workgroup's LDS run in a few launches, requests of
+like size together, the others in one persistent launch of the search in scratch
+memory; all of it is captured in a hipGraph (the first ``run`` plans and captures
+it, later runs replay it; a run whose searches outgrew their room plans the next
+with more). ``autotune`` times candidate shapes of the search in scratch memory
+(workgroup size, resident waves per SIMD, bucket width) on a sample of the
+sources that run there and keeps the fastest.
 
 Each request is prepared exactly as ``NetworkStructure.centrality_shortest``
 prepares it (rust/src/centrality.rs:1624-1874 semantics), so its results equal
@@ -96,7 +99,8 @@ class CentralityBatch:
         _native.check(_native.load().cs_batch_set_tuning(self._h, ctypes.byref(t)))
 
     def autotune(self, sample_fraction: float = 0.03) -> dict:
-        """Time candidate launch shapes on a sample of the sources; keep and return the fastest."""
+        """Time candidate launch shapes on a sample of the sources they are for (those not searched in
+        LDS; none: the shape stays); keep and return the fastest."""
         t = _native.CsTuning()
         _native.check(_native.load().cs_batch_autotune(self._h, float(sample_fraction), ctypes.byref(t)))
         return {name: getattr(t, name) for name, _ in t._fields_}

@@ -13,9 +13,11 @@
 //    together: none of them can reach another's band. When the smallest route
 //    itself is not that far below L (straight continuations cost almost
 //    nothing), it settles alone, which is the serial search's own step.
-//  * The settled states are sorted by their key and their out-edges relax one
-//    per lane, in lane order = settle order. Lanes whose targets are the same
-//    node take turns, lowest lane first.
+//  * The settled states get their positions in the order of the lanes they were
+//    found in, which within a batch is no settle order, and their out-edges
+//    relax one per lane. Lanes whose targets are the same node take turns in
+//    settle order: by the route of the state they leave, then its seconds at
+//    push, then its original number.
 //
 // A lane-per-source search keeps its maps, records and queue in HBM and pays a
 // chain of dependent cache misses per state; here a source's state is a few
@@ -37,7 +39,8 @@
 // over the routes, for the states that precede another only (63% on a lattice).
 //
 // What bounds it: the latency of one batch's instructions and LDS accesses
-// (about 8 states, 27 edges), times the waves a CU's LDS holds. On the dual of
+// (about 8 states, 27 edges; waits are 57% of a wave's cycles on the dual below),
+// times the waves a CU's LDS holds. On the dual of
 // the 150x150 lattice at [500, 1000, 2000] m (32.5k sources, 1,870 states each)
 // 20 KiB per wave run eight waves per CU: 20.2 ms, against 55.1 ms for the
 // lane-per-source kernel; with seconds, lists and page numbers in LDS too (30
@@ -61,7 +64,8 @@ constexpr uint32_t kRow = 4;                  // out-edges of a state's row
 constexpr uint32_t kChunk = kWave / kRow;     // states relaxed together
 constexpr uint32_t kNoEdge = 0xffffffffu;     // padding entry of a row
 constexpr uint32_t kRowSpill = 0xfffffffeu;   // first entry of a row whose edges lie in the spill list {.., begin, count}
-constexpr uint32_t kNearGoal = 56;            // (28, 40, 52: 27.3, 25.1, 24.3 ms on the 150x150 dual) a refill brings the near set up to this many states where routes allow
+constexpr uint32_t kNearGoal = 56;            // a refill brings the near set up to this many states where routes allow
+                                              // (an earlier layout, 24.3 ms on the 150x150 dual: with 28, 40, 52 27.3, 25.1, 24.3)
 constexpr uint32_t kOwn = 128;                // conflict table entries
 constexpr uint32_t kPage = 3;                 // a page: a run of 8 nodes
 constexpr uint32_t kLdsStage = 8 * kOwn, kLdsRoutes = kLdsStage + 16 * kWave;

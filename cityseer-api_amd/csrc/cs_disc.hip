@@ -24,11 +24,11 @@
 //    (centrality.rs:823-873) one (threshold, kind) array per wave, dependencies
 //    in LDS over the distances, for the nodes that precede another only.
 //
-// A round is a chain of LDS and L2 round trips (front, page, distance, offer),
-// three quarters of a wave's cycles are waits; workgroups in flight hide them, so
+// A round is a chain of LDS and L2 round trips (front, page, distance, offer):
+// waits are 75% of a wave's cycles on the city below; workgroups in flight hide them, so
 // the layout counts LDS in the units a CU gives out. Against a wave per source
 // with its state in scratch (cs_search.hip), kernel ms: 32,400 sources, four
-// thresholds to 5,000 m, both measures (reach 3,960) 24.8 -> 19.6; 30,406
+// thresholds to 5,000 m, both measures (reach 3,960) 24.8 -> 19.3; 30,406
 // sources, closeness to 800 m on 20 m pieces (reach 1,003) 3.85 -> 2.42; 676
 // sources to 800 m (reach 93) 0.122 -> 0.079; 64 sources 0.089 -> 0.046.
 #include "cs_internal.hpp"
@@ -1267,6 +1267,7 @@ struct DiscClass {
 };
 
 // Waves of a workgroup: a round settles most of the front, sixteen nodes a wave.
+// (Lines from two workloads:)
 // Front 52 (closeness on 20 m pieces to 800 m): one wave 2.65 ms, two 2.42, four
 // 2.99. Eight towns to 1,600 m: 3.04 ms by this rule, 3.14 with the lines at 64
 // and 160, 3.44 at 24 and 48.

@@ -405,7 +405,8 @@ int cs_get_tuning(cs_tuning *t);
 int cs_release_workspaces(void);
 
 /* A batch of node_centrality_shortest jobs (any graphs, each with its own
- * thresholds and sources) run as one persistent launch captured in a hipGraph.
+ * thresholds and sources) run as one captured hipGraph: a few launches of searches
+ * in LDS, jobs of like size together, and one persistent launch of the others.
  * Graphs must outlive the batch. Not thread-safe: one thread drives a batch. */
 typedef struct cs_batch cs_batch;
 int cs_batch_create(cs_batch **out);
@@ -415,8 +416,9 @@ void cs_batch_destroy(cs_batch *b);
  * filled by cs_batch_results. Returns the job index (>= 0, in call order) or
  * minus a status code. */
 int cs_batch_add_shortest(cs_batch *b, cs_graph *g, const cs_params *p, double *out, uint32_t *reach_totals);
-/* Times candidate launch shapes on a `sample_fraction` of the batch's sources
- * and keeps the fastest; `chosen` (may be NULL) receives it. */
+/* Times candidate launch shapes on a `sample_fraction` of the sources they are
+ * for, those that do not search in LDS, and keeps the fastest (none: the shape
+ * stays); `chosen` (may be NULL) receives it. */
 int cs_batch_autotune(cs_batch *b, double sample_fraction, cs_tuning *chosen);
 int cs_batch_set_tuning(cs_batch *b, const cs_tuning *t);
 /* Runs every job: the first run uploads the jobs and captures the launch,
