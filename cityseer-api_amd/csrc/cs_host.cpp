@@ -573,6 +573,57 @@ struct KeptBuf {
   }
 };
 
+// Pinned host buffers kept the same way: a copy into pageable memory takes 23 us
+// at 8 kB and 113 at 256, into one of these and on 13 and 19; past 4 MB there is
+// no difference.
+struct KeptPinned {
+  static constexpr size_t kMost = 4u << 20, kMostBufs = 4;
+  struct Pool {
+    std::mutex mu;
+    std::vector<std::pair<size_t, char *>> free;
+    void release() {
+      std::lock_guard<std::mutex> lk(mu);
+      for (auto &x : free) (void)hipHostFree(x.second);
+      free.clear();
+    }
+  };
+  static Pool &pool() {
+    static Pool *p = new Pool;  // (outlives the runtime's own teardown)
+    return *p;
+  }
+  char *p = nullptr;
+  size_t bytes = 0;
+  int errors = std::uncaught_exceptions();
+  explicit KeptPinned(size_t need) {
+    for (bytes = 64u << 10; bytes < need;) bytes *= 2;
+    Pool &k = pool();
+    {
+      std::lock_guard<std::mutex> lk(k.mu);
+      for (size_t i = 0; i < k.free.size() && !p; ++i)
+        if (k.free[i].first >= need) {
+          bytes = k.free[i].first;
+          p = k.free[i].second;
+          k.free[i] = k.free.back();
+          k.free.pop_back();
+        }
+    }
+    if (!p) hip_check(hipHostMalloc(reinterpret_cast<void **>(&p), bytes, hipHostMallocDefault), "hipHostMalloc");
+  }
+  ~KeptPinned() {
+    Pool &k = pool();
+    if (std::uncaught_exceptions() <= errors) {
+      std::lock_guard<std::mutex> lk(k.mu);
+      if (k.free.size() < kMostBufs) {
+        k.free.emplace_back(bytes, p);
+        return;
+      }
+    }
+    (void)hipHostFree(p);
+  }
+  KeptPinned(const KeptPinned &) = delete;
+  KeptPinned &operator=(const KeptPinned &) = delete;
+};
+
 struct KeptStream {
   hipStream_t s = nullptr;
   int dev = 0, errors = std::uncaught_exceptions();
@@ -1914,6 +1965,7 @@ int cs_release_workspaces(void) {
   return guarded([] {
     release_search_workspaces();
     kept().release();
+    KeptPinned::pool().release();
     release_angular_workspaces();
   });
 }
@@ -2021,7 +2073,6 @@ int cs_batch_results(cs_batch *b) {
   return guarded([&] {
     if (!b) fail(CS_EINVAL, "batch must not be NULL");
     if (!b->have_results) fail(CS_EINVAL, "the batch has no results: call cs_batch_run first");
-    std::vector<uint32_t> hreach(8 * b->jobs.size());
     const struct OnDevice {  // the batch's, whichever is current
       int was = 0;
       explicit OnDevice(int dev) {
@@ -2030,24 +2081,61 @@ int cs_batch_results(cs_batch *b) {
       }
       ~OnDevice() { (void)hipSetDevice(was); }
     } on(b->device);
-    size_t most = 0;
-    for (const cs_batch::JobHost &j : b->jobs) most = std::max(most, (size_t)7 * j.spec.T * j.h->g.n);
-    KeptBuf tmp(8 * most);
-    if (!hreach.empty())
+    // results up to 4 MB come back together, each job's put in order on the
+    // device and one copy for all: a copy and its wait per job took six towns of
+    // 11x11 to 32x32 0.17 ms more than one copy of unordered rows. Larger ones
+    // by themselves.
+    std::vector<uint32_t> hreach(8 * b->jobs.size(), 0);
+    bool tracked = false;
+    size_t most = 0, small = 0;
+    auto bytes_of = [](const cs_batch::JobHost &j) { return 8 * (size_t)7 * j.spec.T * j.h->g.n; };
+    for (const cs_batch::JobHost &j : b->jobs) {
+      tracked = tracked || j.spec.track_reach;
+      if (bytes_of(j) <= KeptPinned::kMost) small += bytes_of(j);
+      else most = std::max(most, bytes_of(j));
+    }
+    const size_t room = std::min(small, KeptPinned::kMost);
+    KeptBuf tmp(std::max(most, room));
+    KeptPinned host(std::max<size_t>(room, 1));
+    if (tracked)  // (nothing counted otherwise)
       hip_check(hipMemcpy(hreach.data(), b->d_reach, 4 * hreach.size(), hipMemcpyDeviceToHost), "copy out");
+    auto perm_of = [&](const cs_batch::JobHost &j) -> const uint32_t * {
+      if (j.h->g.identity_order) return nullptr;
+      std::lock_guard<std::mutex> lk(j.h->g.mu);
+      return device_graph(j.h->g, b->device).perm;
+    };
+    std::vector<size_t> waiting;  // jobs in the buffer, not yet copied out
+    size_t used = 0;
+    auto flush = [&] {
+      if (waiting.empty()) return;
+      hip_check(hipMemcpyAsync(host.p, tmp.p, used, hipMemcpyDeviceToHost, b->stream), "copy out");
+      hip_check(hipStreamSynchronize(b->stream), "sync");
+      const char *from = host.p;
+      for (const size_t i : waiting) {
+        const cs_batch::JobHost &j = b->jobs[i];
+        const size_t N = j.h->g.n, rows = 8 * (size_t)j.spec.T * N;
+        for (uint32_t m = 0; m < 7; ++m, from += rows) std::memcpy(j.out + ((size_t)m * j.out_T + j.t0) * N, from, rows);
+      }
+      waiting.clear();
+      used = 0;
+    };
     for (size_t i = 0; i < b->jobs.size(); ++i) {
       const cs_batch::JobHost &j = b->jobs[i];
-      const uint32_t N = j.h->g.n, T = j.spec.T;
-      const uint32_t *d_perm = nullptr;
-      if (!j.h->g.identity_order) {
-        std::lock_guard<std::mutex> lk(j.h->g.mu);
-        d_perm = device_graph(j.h->g, b->device).perm;
-      }
-      results_out(b->d_acc + j.acc_off, N, 7, T, b->NT, d_perm, 5, 6, j.betw ? j.betw_scale : 1.0, tmp.as<double>(), j.out,
-                  b->stream, j.out_T, j.t0);
       if (j.reach)
-        for (uint32_t t = 0; t < T; ++t) j.reach[j.t0 + t] = hreach[8 * i + t];
+        for (uint32_t t = 0; t < j.spec.T; ++t) j.reach[j.t0 + t] = hreach[8 * i + t];
+      const size_t bytes = bytes_of(j);
+      if (!bytes || bytes > KeptPinned::kMost) continue;
+      if (used + bytes > room) flush();
+      results_ordered(b->d_acc + j.acc_off, j.h->g.n, 7, j.spec.T, b->NT, perm_of(j), 5, 6, j.betw ? j.betw_scale : 1.0,
+                      reinterpret_cast<double *>(tmp.as<char>() + used), b->stream);
+      waiting.push_back(i);
+      used += bytes;
     }
+    flush();
+    for (const cs_batch::JobHost &j : b->jobs)
+      if (bytes_of(j) > KeptPinned::kMost)
+        results_out(b->d_acc + j.acc_off, j.h->g.n, 7, j.spec.T, b->NT, perm_of(j), 5, 6, j.betw ? j.betw_scale : 1.0,
+                    tmp.as<double>(), j.out, b->stream, j.out_T, j.t0);
     hip_check(hipStreamSynchronize(b->stream), "sync");
   });
 }

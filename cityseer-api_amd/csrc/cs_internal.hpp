@@ -370,6 +370,10 @@ void results_out(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32
                  uint32_t m0, uint32_t m1, double scale, double *d_tmp, double *out, hipStream_t stream, uint32_t out_T = 0,
                  uint32_t t0 = 0);
 
+// The same into a device buffer [M][T][N].
+void results_ordered(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32_t stride, const uint32_t *d_perm,
+                     uint32_t m0, uint32_t m1, double scale, double *d_out, hipStream_t stream);
+
 struct ShortestBatch;
 ShortestBatch *batch_new(std::vector<JobSpec> specs, std::vector<ZeroRegion> zero, uint32_t NT, int device,
                          const Tuning &tune);

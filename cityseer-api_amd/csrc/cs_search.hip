@@ -2657,6 +2657,15 @@ __global__ void k_results(double *dst, const double *src, const uint32_t *perm, 
   dst[(size_t)row * N + v] = x;
 }
 
+void results_ordered(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32_t stride, const uint32_t *d_perm,
+                     uint32_t m0, uint32_t m1, double scale, double *d_out, hipStream_t stream) {
+  if (!N || !M || !T) return;
+  for (uint32_t row = 0; row < M * T; row += 32768)
+    hipLaunchKernelGGL(k_results, dim3((N + 255) / 256, std::min(M * T - row, 32768u)), dim3(256), 0, stream, d_out, d_acc,
+                       d_perm, N, T, stride, m0, m1, scale, row);
+  hip_check(hipGetLastError(), "k_results launch");
+}
+
 void results_out(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32_t stride, const uint32_t *d_perm,
                  uint32_t m0, uint32_t m1, double scale, double *d_tmp, double *out, hipStream_t stream, uint32_t out_T,
                  uint32_t t0) {
@@ -2664,10 +2673,7 @@ void results_out(const double *d_acc, uint32_t N, uint32_t M, uint32_t T, uint32
   if (out_T == 0) out_T = T;
   const double *from = d_acc;
   if (d_perm || stride != T || scale != 1.0) {
-    for (uint32_t row = 0; row < M * T; row += 32768)
-      hipLaunchKernelGGL(k_results, dim3((N + 255) / 256, std::min(M * T - row, 32768u)), dim3(256), 0, stream, d_tmp, d_acc,
-                         d_perm, N, T, stride, m0, m1, scale, row);
-    hip_check(hipGetLastError(), "k_results launch");
+    results_ordered(d_acc, N, M, T, stride, d_perm, m0, m1, scale, d_tmp, stream);
     from = d_tmp;
   }
   const size_t rows = (size_t)T * N;

@@ -169,3 +169,17 @@ def test_batch_of_more_cutoffs_than_a_graph_keeps():
     res = b.results()
     for k in (0, 35, 69):
         _check_equal(res[k], ns.centrality_shortest(distances=[dists[k]]), [dists[k]], f"request {k}")
+
+
+def test_results_of_all_sizes_come_back():
+    """Results past 4 MB by themselves, smaller ones together, more of them than one buffer holds."""
+    nets = [mock.network_structure_from_lattice(mock.perturbed_lattice(s, seed=s)) for s in (5, 200, 90, 12, 95, 100, 7)]
+    dists = [[300], [200, 400], [150, 250, 350, 450], [100 * k for k in range(1, 11)], [300], [250, 500], [400]]
+    b = CentralityBatch()
+    for ns, d in zip(nets, dists):
+        b.add_shortest(ns, distances=d)
+    for rep in range(2):
+        say(f"results of {len(nets)} networks, run {rep}")
+        b.run()
+        for i, (ns, d, r) in enumerate(zip(nets, dists, b.results())):
+            _check_equal(r, ns.centrality_shortest(distances=d), d, f"network {i}")
