@@ -226,6 +226,7 @@ _SIGNATURES = {
     "cs_batch_set_tuning": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(CsTuning)]),
     "cs_batch_run": (ctypes.c_int, [ctypes.c_void_p]),
     "cs_batch_results": (ctypes.c_int, [ctypes.c_void_p]),
+    "cs_batch_results_into": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]),
     "cs_server_create": (ctypes.c_int, [ctypes.POINTER(CsServerConfig), ctypes.POINTER(ctypes.c_void_p)]),
     "cs_server_destroy": (None, [ctypes.c_void_p]),
     "cs_server_submit": (

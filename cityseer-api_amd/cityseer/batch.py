@@ -112,13 +112,15 @@ class CentralityBatch:
 
     def results(self) -> list[_res.CentralityShortestResult]:
         """Copy the last run's results out, one result object per job in insertion order."""
-        _native.check(_native.load().cs_batch_results(self._h))
+        outs = [np.empty_like(j["out"]) for j in self._jobs]
+        at = (ctypes.c_void_p * max(len(outs), 1))(*(o.ctypes.data for o in outs))
+        _native.check(_native.load().cs_batch_results_into(self._h, at))
         res = []
-        for j in self._jobs:
+        for j, out in zip(self._jobs, outs):
             ns, plan, t = j["ns"], j["plan"], j["t"]
             res.append(
                 _res.CentralityShortestResult(
-                    j["dists"], ns.node_keys_py(), ns.node_indices(), j["out"].copy(),
+                    j["dists"], ns.node_keys_py(), ns.node_indices(), out,
                     j["reach"][:t].tolist() if plan["track"] else [], plan["sampled"] if plan["track"] else 0,
                 )
             )

@@ -825,6 +825,7 @@ struct cs_batch {
     bool betw = false;
     double betw_scale = 1.0;
     size_t acc_off = 0;
+    uint32_t request = 0;
     uint32_t out_T = 0, t0 = 0;  // the request's thresholds; this job's first (a chunk of at most kMaxT)
   };
   int device = -1;
@@ -2022,6 +2023,7 @@ int cs_batch_add_shortest(cs_batch *b, cs_graph *h, const cs_params *p, double *
     }
     b->drop_device();
     for (auto &j : chunks) {
+      j.request = (uint32_t)b->n_requests;
       b->NT = std::max(b->NT, j.spec.T);
       b->jobs.push_back(std::move(j));
     }
@@ -2069,7 +2071,9 @@ int cs_batch_run(cs_batch *b) {
   return rc;
 }
 
-int cs_batch_results(cs_batch *b) {
+int cs_batch_results(cs_batch *b) { return cs_batch_results_into(b, nullptr); }
+
+int cs_batch_results_into(cs_batch *b, double *const *outs) {
   return guarded([&] {
     if (!b) fail(CS_EINVAL, "batch must not be NULL");
     if (!b->have_results) fail(CS_EINVAL, "the batch has no results: call cs_batch_run first");
@@ -2104,6 +2108,7 @@ int cs_batch_results(cs_batch *b) {
       std::lock_guard<std::mutex> lk(j.h->g.mu);
       return device_graph(j.h->g, b->device).perm;
     };
+    auto out_of = [&](const cs_batch::JobHost &j) { return outs ? outs[j.request] : j.out; };
     std::vector<size_t> waiting;  // jobs in the buffer, not yet copied out
     size_t used = 0;
     auto flush = [&] {
@@ -2114,7 +2119,7 @@ int cs_batch_results(cs_batch *b) {
       for (const size_t i : waiting) {
         const cs_batch::JobHost &j = b->jobs[i];
         const size_t N = j.h->g.n, rows = 8 * (size_t)j.spec.T * N;
-        for (uint32_t m = 0; m < 7; ++m, from += rows) std::memcpy(j.out + ((size_t)m * j.out_T + j.t0) * N, from, rows);
+        for (uint32_t m = 0; m < 7; ++m, from += rows) std::memcpy(out_of(j) + ((size_t)m * j.out_T + j.t0) * N, from, rows);
       }
       waiting.clear();
       used = 0;
@@ -2135,7 +2140,7 @@ int cs_batch_results(cs_batch *b) {
     for (const cs_batch::JobHost &j : b->jobs)
       if (bytes_of(j) > KeptPinned::kMost)
         results_out(b->d_acc + j.acc_off, j.h->g.n, 7, j.spec.T, b->NT, perm_of(j), 5, 6, j.betw ? j.betw_scale : 1.0,
-                    tmp.as<double>(), j.out, b->stream, j.out_T, j.t0);
+                    tmp.as<double>(), out_of(j), b->stream, j.out_T, j.t0);
     hip_check(hipStreamSynchronize(b->stream), "sync");
   });
 }

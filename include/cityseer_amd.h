@@ -426,6 +426,8 @@ int cs_batch_set_tuning(cs_batch *b, const cs_tuning *t);
 int cs_batch_run(cs_batch *b);
 /* Copies the last run's results into the jobs' `out` / `reach_totals` arrays. */
 int cs_batch_results(cs_batch *b);
+/* The same into outs[job index] ([7][T][N] each, in place of the jobs' `out`). */
+int cs_batch_results_into(cs_batch *b, double *const *outs);
 
 /* ---------------------------------------------------------------------- */
 /* Serving: a request loop with continuous batching                       */

@@ -6,6 +6,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+from cityseer import _native
 from cityseer.batch import CentralityBatch
 from cityseer.tools import io, mock
 from oracle.oracle import OracleGraph
@@ -178,8 +179,18 @@ def test_results_of_all_sizes_come_back():
     b = CentralityBatch()
     for ns, d in zip(nets, dists):
         b.add_shortest(ns, distances=d)
+    plain = [ns.centrality_shortest(distances=d) for ns, d in zip(nets, dists)]
+    kept = []
     for rep in range(2):
         say(f"results of {len(nets)} networks, run {rep}")
         b.run()
-        for i, (ns, d, r) in enumerate(zip(nets, dists, b.results())):
-            _check_equal(r, ns.centrality_shortest(distances=d), d, f"network {i}")
+        kept.append(b.results())
+    for res in kept:  # (each call's own arrays)
+        for i, (d, r, p) in enumerate(zip(dists, res, plain)):
+            _check_equal(r, p, d, f"network {i}")
+    assert kept[0][1]._values is not kept[1][1]._values
+    # into the arrays given with the requests, as the C interface has it
+    lib = _native.load()
+    _native.check(lib.cs_batch_results(b._h))
+    for j, r in zip(b._jobs, kept[1]):
+        assert np.array_equal(j["out"], r._values)
