@@ -1256,6 +1256,7 @@ struct DiscClass {
   DiscArgs a;
   uint32_t lds = 0, waves = 1, NT = 1, N = 0;
   bool betw = false;
+  bool again = false;  // searches that ran out of room before
   double room = 1.0;
   double most = 0.0, all = 0.0;  // expected time of its slowest search, of all its searches one by one (ms)
   double load = 0.0;             // `all` on the workgroups the device holds
@@ -1658,10 +1659,11 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
     for (uint32_t i = 0; i < n_failed; ++i) left[i] = d.items.empty() ? make_uint2(0u, fl[i]) : d.items[fl[i]];
     st.retries += n_failed;
     // (a few searched twice cost less than room for them in every workgroup)
-    if (!cap && (uint64_t)n_failed * 32 > d.n)
+    if (!cap && !d.again && (uint64_t)n_failed * 32 > d.n)
       for (const uint32_t i : d.which) (void)disc_more_room(*specs[i].de, specs[i].cs.maxsec, specs[i].g->n);
     // again with more room while LDS has it
     DiscClass e = d;
+    e.again = true;
     e.items = left;
     e.n = n_failed;
     bool wider = false;

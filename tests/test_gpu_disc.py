@@ -183,6 +183,19 @@ def test_batch_of_small_towns_is_one_launch():
                 assert_close(got, alone[i], f"town {i}, run {k}")
 
 
+def test_few_that_outgrow_their_room_cost_the_others_nothing():
+    """A knot of one source in forty-five, which needs several tries: later calls keep their room."""
+    ns = mock.network_structure_from_lattice(_knot(160, 24))
+    seen = []
+    for k in range(4):
+        say(f"call {k} on a network with a small knot")
+        res = stack(ns.centrality_shortest(distances=[150, 300]), SHORTEST_KEYS, [150, 300])
+        seen.append((_native.last_stats()["retries"], res))
+        assert np.array_equal(res[0], seen[0][1][0])
+        assert_close(res, seen[0][1], f"call {k}")
+    assert seen[0][0] > 0 and all(r == seen[0][0] for r, _ in seen), [r for r, _ in seen]
+
+
 def test_batch_learns_the_room_its_searches_take():
     """Runs of a batch whose knot outgrows the probed searches (1,296 nodes to their 75): each plans the next
     with more room, until none searches twice; every run the same."""
