@@ -1256,7 +1256,11 @@ struct DiscClass {
   DiscArgs a;
   uint32_t lds = 0, waves = 1, NT = 1, N = 0;
   bool betw = false;
-  bool again = false;  // searches that ran out of room before
+  // searches that ran out of room before: the first launch's searches, workgroups
+  // and time, and the time of the tries since
+  bool again = false;
+  uint32_t first_n = 0, first_blocks = 0;
+  double first_ms = 0.0, tries_ms = 0.0;
   double room = 1.0;
   double most = 0.0, all = 0.0;  // expected time of its slowest search, of all its searches one by one (ms)
   double load = 0.0;             // `all` on the workgroups the device holds
@@ -1593,9 +1597,31 @@ static void disc_enqueue(const DiscClass &d, uint32_t blocks, hipStream_t stream
   else hipLaunchKernelGGL(k_disc<8>, grid, block, d.lds, stream, d.a);
 }
 
+// The tries of a request's searches ended with room for all. Later calls give it
+// to every search from the start where the workgroups that costs are expected to
+// cost less time than the tries took.
+static void disc_learn(const DiscClass &d, const JobSpec &js, uint32_t cus) {
+  DiscClass g = disc_pair(d, d);
+  auto up = [&](uint32_t x, uint32_t most) { return (uint32_t)std::min<double>(most, std::ceil(x * d.room)); };
+  g.reach.nodes = up(d.reach.nodes, d.N);
+  g.reach.front = up(d.reach.front, d.N);
+  g.reach.inner = up(d.reach.inner, d.N);
+  for (uint32_t ps = 4; ps < kProbePages; ++ps) g.reach.pages[ps] = up(d.reach.pages[ps], (d.N + (1u << ps) - 1) >> ps);
+  if (!disc_estimate(g, 0, cus)) return;
+  const double had = std::min(d.first_n, d.first_blocks);
+  const double has = std::min(d.first_n, cus * std::max(1u, std::min(blocks_by_lds(g.lds), 20u / g.waves)));
+  if (d.first_ms * (had / has - 1.0) > d.tries_ms) return;
+  std::lock_guard<std::mutex> lk(js.de->disc_mu);
+  const auto it = js.de->disc->reach.find(js.cs.maxsec);
+  if (it != js.de->disc->reach.end() && it->second.nodes <= g.reach.nodes) it->second = g.reach;
+}
+
 bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, hipStream_t stream, cs_stats &st,
                  uint32_t *progress, std::vector<uint2> *rest) {
   const int dev = specs[0].dg->device;
+  int n_cu = 0;
+  hip_check(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev), "attribute");
+  const uint32_t cus = (uint32_t)n_cu;
   DiscWorkspace *ws = acquire_disc(dev);
   std::lock_guard<std::mutex> guard(ws->mu, std::adopt_lock);
   std::vector<DiscClass> work = disc_plan(specs, NT, cap, ws->tmp, stream, rest);
@@ -1651,28 +1677,39 @@ bool launch_disc(const std::vector<JobSpec> &specs, uint32_t NT, uint32_t cap, h
     st.within_sum += stv[2];
     const uint32_t n_failed = h[kXcd];
     thread_lds_searches() += d.n - n_failed;
-    if (!n_failed) continue;
+    if (d.again) {
+      d.tries_ms += ms;
+    } else {
+      d.first_n = d.n;
+      d.first_blocks = blocks;
+      d.first_ms = ms;
+    }
+    if (!n_failed) {
+      if (d.again && !cap && d.which.size() == 1) disc_learn(d, specs[d.which[0]], cus);
+      continue;
+    }
     if (h[kXcd + 1] & kFailInternal) fail(CS_EINTERNAL, "search invariant violated (settle order)");
     std::vector<uint32_t> fl(n_failed);
     hip_check(hipMemcpy(fl.data(), fail_list, 4ull * n_failed, hipMemcpyDeviceToHost), "copy");
     std::vector<uint2> left(n_failed);
     for (uint32_t i = 0; i < n_failed; ++i) left[i] = d.items.empty() ? make_uint2(0u, fl[i]) : d.items[fl[i]];
     st.retries += n_failed;
-    // (a few searched twice cost less than room for them in every workgroup)
-    if (!cap && !d.again && (uint64_t)n_failed * 32 > d.n)
-      for (const uint32_t i : d.which) (void)disc_more_room(*specs[i].de, specs[i].cs.maxsec, specs[i].g->n);
-    // again with more room while LDS has it
+    // again with more room while LDS has it: as much as leaves them all running
+    // at once, or half as much again
     DiscClass e = d;
     e.again = true;
     e.items = left;
     e.n = n_failed;
     bool wider = false;
-    for (double f = d.room * 1.5; f < 40.0 && !wider; f *= 1.5) {
+    double room = d.room;
+    for (double f = d.room * 1.5; f < 40.0; f *= 1.5) {
       e.room = f;
       uint32_t b = 0;
-      if (!disc_shape(e, cap, dev, false, &b)) break;
-      wider = e.a.S > d.a.S || e.a.P > d.a.P || e.a.F > d.a.F;
+      if (!disc_shape(e, cap, dev, false, &b) || (wider && b < n_failed)) break;
+      wider = wider || e.a.S > d.a.S || e.a.P > d.a.P || e.a.F > d.a.F;
+      room = f;
     }
+    e.room = room;
     if (wider && !cap) {
       work.push_back(std::move(e));
     } else {
