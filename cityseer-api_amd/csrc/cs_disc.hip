@@ -1153,6 +1153,7 @@ void disc_probe(const std::vector<const JobSpec *> &asked, DevVec &tmp, hipStrea
         const uint32_t *o = &h[(i * kProbes + q) * kProbeWords];
         r.nodes = std::max(r.nodes, o[0]);
         r.front = std::max(r.front, o[1]);
+        if (q + 1 < kProbes) r.spread = std::max(r.spread, o[1]);
         r.inner = std::max(r.inner, o[2]);
         for (uint32_t ps = 4; ps < kProbePages; ++ps) r.pages[ps] = std::max(r.pages[ps], o[ps - 1]);
       }
@@ -1275,7 +1276,9 @@ struct DiscClass {
 // (Lines from two workloads:)
 // Front 52 (closeness on 20 m pieces to 800 m): one wave 2.65 ms, two 2.42, four
 // 2.99. Eight towns to 1,600 m: 3.04 ms by this rule, 3.14 with the lines at 64
-// and 160, 3.44 at 24 and 48.
+// and 160, 3.44 at 24 and 48. (The front of a town's middle, which only its few
+// nearest sources have, is not what they are about: with it 3,095 sources to
+// 2,750 m on a 62x62 town take four waves and 0.68 ms, without it two and 0.59.)
 static uint32_t disc_waves(uint32_t front) { return front <= 40 ? 1u : front <= 100 ? 2u : 4u; }
 
 // ... as far as the request itself tells.
@@ -1450,7 +1453,7 @@ static std::vector<DiscClass> disc_plan(const std::vector<JobSpec> &specs, uint3
       std::memset(&a, 0, sizeof(a));
       if (!w.reach.count(js.cs.maxsec)) disc_probe({&js}, tmp, stream);  // (forgotten over more than 64 others)
       r = w.reach.at(js.cs.maxsec);
-      waves = disc_waves(r.front);
+      waves = disc_waves(r.spread);
       if (!disc_layout(a, js.g->n, r, js.cs.betweenness, waves, 1.0, cap, &lds)) continue;
     }
     if (!disc_pays(lds, waves, js.cs.betweenness, js.n_sources, cus)) continue;

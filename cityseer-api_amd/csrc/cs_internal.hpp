@@ -105,6 +105,7 @@ struct DiscGraph {
   // that precede another
   struct Reach {
     uint32_t nodes = 0, front = 0, inner = 0;
+    uint32_t spread = 0;  // `front` of the sources spread over the node order
     uint32_t pages[10] = {0};
   };
   std::map<float, Reach> reach;

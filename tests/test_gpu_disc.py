@@ -123,6 +123,17 @@ def test_city_is_searched_once():
     assert _native.last_stats()["retries"] == 0 and _native.last_lds_searches() == ns.node_count()
 
 
+def test_waves_of_a_town_as_wide_as_its_searches():
+    """Two waves a workgroup: only the town's middle has a front past their line (100), its spread sources none."""
+    ns = mock.network_structure_from_lattice(mock.perturbed_lattice(56, seed=2, diag_frac=0.05))
+    n = ns.node_count() // 2  # all at once: 2 waves each, 4 by the middle's front
+    src = np.linspace(0, ns.node_count() - 1, n).astype(int).tolist()
+    say(f"{ns.node_count()} nodes, {n} sources to 2,750 m")
+    ns.centrality_shortest(distances=[2750], source_indices=src)
+    stats = _native.last_stats()
+    assert _native.last_lds_searches() == n and stats["waves"] == 2 * n, stats
+
+
 def test_large_reach_is_searched_once():
     """Too large for a workgroup's LDS and for the usual records of a wave: no source is searched twice."""
     O.set_heap_mode(False)
