@@ -1,7 +1,8 @@
 // cs_angular.hip -- simplest-path (angular) centrality on the dual graph, one
 // lane per source: what the LDS search (cs_angwave.hip) does not take or has no
 // room for (tolerances above the tie band, searches of thousands of nodes,
-// negative increments), the single-source tree and the reach lists.
+// negative increments, many sources whose waves would take turns), the
+// single-source tree and the reach lists.
 //
 // Angular route increments are turn angles plus 1e-6 x length
 // (centrality.rs:665-667): straight continuations cost almost nothing, so no

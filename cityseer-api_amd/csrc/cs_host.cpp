@@ -2077,6 +2077,9 @@ int cs_batch_results_into(cs_batch *b, double *const *outs) {
   return guarded([&] {
     if (!b) fail(CS_EINVAL, "batch must not be NULL");
     if (!b->have_results) fail(CS_EINVAL, "the batch has no results: call cs_batch_run first");
+    if (outs)
+      for (const cs_batch::JobHost &j : b->jobs)
+        if (!outs[j.request]) fail(CS_EINVAL, "outs must not hold NULL");
     const struct OnDevice {  // the batch's, whichever is current
       int was = 0;
       explicit OnDevice(int dev) {

@@ -3,6 +3,8 @@ plain one-call-per-request path and the oracle, on every replay and after autotu
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -194,3 +196,5 @@ def test_results_of_all_sizes_come_back():
     _native.check(lib.cs_batch_results(b._h))
     for j, r in zip(b._jobs, kept[1]):
         assert np.array_equal(j["out"], r._values)
+    with pytest.raises(ValueError, match="outs"):
+        _native.check(lib.cs_batch_results_into(b._h, (ctypes.c_void_p * len(nets))()))
